@@ -98,10 +98,27 @@ struct RParams {
 
 // A window is a run of whole sample passes of one or more jobs; part k
 // holds passes [pass0, pass0 + npass) of job `job` at window samples
-// [off, off + npass * npix), pass-major.
+// [off, off + npass * npix): all passes of a pixel together, pixels in the
+// tile order below.  So the 64 paths a wave starts with share a pixel (at 64
+// samples per pixel) or a few neighbouring ones: their camera rays walk the
+// same nodes, hit the same triangles and materials, and their first shadow
+// rays run side by side.  Against whole passes of the image in row order
+// the 1080p x 64 frame of 1.31 M triangles went from 326 to 298 ms, a batch
+// of eight small scenes from 46.8 to 35.4 ms.
 struct PartDev {
-    int job, pass0, off, npix, npass, pad[3];
+    int job, pass0, off, npix, npass, width, pad[2];
 };
+
+// Pixel order of a window's samples: strips of 8 rows, column by column
+// inside a strip (64 consecutive pixels are an 8 x 8 tile); the last strip
+// takes the rows that are left.
+constexpr int kStripRows = 8;
+RT_HD int pixel_of_rank(int q, int W, int npix) {
+    const int strip = q / (kStripRows * W), y0 = strip * kStripRows;
+    const int r = q - y0 * W, left = npix / W - y0, h = left < kStripRows ? left : kStripRows;
+    const int x = r / h;
+    return (y0 + r - x * h) * W + x;
+}
 
 // Batch job on the device: its scene view and render parameters.
 struct JobDev {
@@ -297,11 +314,16 @@ __device__ __forceinline__ int pf_cat(int32_t f) { return (f >> kPfCatShift) & 3
 __device__ __forceinline__ int pf_pend(int32_t f) { return (f >> kPfPendShift) & 0xff; }
 
 // XCD-aware block order: gfx950 dispatches consecutive workgroups round-robin
-// over its 8 XCDs; renumber so each XCD walks one contiguous range of the
-// queue (neighbouring rays share BVH nodes in that XCD's L2).
+// over its 8 XCDs; renumber so each XCD walks runs of kXcdRun consecutive
+// blocks (neighbouring rays share BVH nodes in that XCD's L2) while the eight
+// stay side by side in the queue, so sky and object parts of the image load
+// them evenly (one eighth of the pool per XCD ran that frame in 349 ms).
+constexpr uint32_t kXcdRun = 32;
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb) {
-    uint32_t q = nb / 8u, r = nb % 8u, x = b % 8u;
-    return x * q + min(x, r) + b / 8u;
+    const uint32_t whole = nb / (8u * kXcdRun) * (8u * kXcdRun);
+    if (b >= whole) return b;   // the last, partial round keeps its order
+    const uint32_t x = b % 8u, i = b / 8u;
+    return (i / kXcdRun * 8u + x) * kXcdRun + i % kXcdRun;
 }
 __device__ __forceinline__ uint32_t xcd_block() { return xcd_remap(blockIdx.x, gridDim.x); }
 
@@ -935,10 +957,10 @@ __device__ __forceinline__ void resolve_sample(const PathBufs& P, int sid, int& 
         else hi = mid - 1;
     }
     const PartDev pt = P.parts[lo];
-    int local = sid - pt.off;
+    const int local = sid - pt.off, q = local / pt.npass;
     job = pt.job;
-    pix = local % pt.npix;
-    pass = pt.pass0 + local / pt.npix;
+    pix = pixel_of_rank(q, pt.width, pt.npix);
+    pass = pt.pass0 + local - q * pt.npass;
 }
 
 // Starts the camera path of window sample `sid` (pixel `pix`, sample pass
@@ -2335,15 +2357,15 @@ __global__ void __launch_bounds__(kBlock) k_retire(JOBS jobs, PathBufs P) {
 // CaptureAccumulator.Add, Renderer.cs:829-856): the window's samples of a
 // pixel are summed pass by pass, even passes into half A, odd into half B.
 __global__ void __launch_bounds__(kBlock) k_accum(RParams R, PathBufs P, FilmBufs F, int pass0, int passes, int off) {
-    int pix = blockIdx.x * kBlock + threadIdx.x;
-    if (pix >= R.npix) return;
-    const int np = R.npix;
+    const int q = blockIdx.x * kBlock + threadIdx.x;
+    if (q >= R.npix) return;
+    const int np = R.npix, pix = pixel_of_rank(q, R.W, np);
     f3 sum = mk(F.sum[pix], F.sum[np + pix], F.sum[2 * np + pix]);
     f3 sa = mk(F.sa[pix], F.sa[np + pix], F.sa[2 * np + pix]);
     f3 sb = mk(F.sb[pix], F.sb[np + pix], F.sb[2 * np + pix]);
     for (int sl = 0; sl < passes; sl++) {
         int s = R.soff + pass0 + sl;
-        int64_t k = (int64_t)off + (int64_t)sl * np + pix;
+        int64_t k = (int64_t)off + (int64_t)q * passes + sl;
         float4 l = P.res_l[k];
         f3 L = f3of(l);
         sum += L;
@@ -3911,7 +3933,7 @@ int rt_render(rt_ctx* ctx, const rt_scene* sc, const rt_settings* s, const rt_fi
     WindowPlan plan;
     for (int base = 0; base < spp; base += K) {
         const int passes = std::min(K, spp - base);
-        plan.add_window({PartDev{0, base, 0, npix, passes, {0, 0, 0}}}, passes * npix);
+        plan.add_window({PartDev{0, base, 0, npix, passes, s->width, {0, 0}}}, passes * npix);
     }
     LoopTiming tm;
     OneJob one{S, R};
@@ -4014,7 +4036,7 @@ int rt_adjoint(rt_ctx* ctx, const rt_scene* sc, const rt_settings* s, const floa
         for (int base = 0; base < spp; base += K) {
             const int passes = std::min(K, spp - base);
             WindowPlan plan;
-            plan.add_window({PartDev{0, base, 0, npix, passes, {0, 0, 0}}}, passes * npix);
+            plan.add_window({PartDev{0, base, 0, npix, passes, s->width, {0, 0}}}, passes * npix);
             P.adj_pass = 1;
             rc = run_windows(ctx, one, P, maxs, true, false, sc->stack_depth, nullptr, nullptr, plan, no_accum,
                              tm_primal);
@@ -4112,7 +4134,7 @@ int rt_render_batch(rt_ctx* ctx, const rt_batch_job* jobs, int32_t n_jobs, int32
                 if ((int64_t)K * npix > (1ll << 31) - 1) return fail(ctx, RT_ERR_INVALID_ARGUMENT, "image too large");
                 for (int base = 0; base < spp; base += K) {
                     const int passes = std::min(K, spp - base);
-                    sg.plan.add_window({PartDev{j, base, 0, (int)npix, passes, {0, 0, 0}}}, passes * (int)npix);
+                    sg.plan.add_window({PartDev{j, base, 0, (int)npix, passes, st->width, {0, 0}}}, passes * (int)npix);
                 }
                 segs.push_back(sg);
                 continue;
@@ -4128,7 +4150,7 @@ int rt_render_batch(rt_ctx* ctx, const rt_batch_job* jobs, int32_t n_jobs, int32
                 }
                 int np = (int)std::max<int64_t>(1, std::min<int64_t>(room, spp - pass));
                 if (used + np * npix > (1ll << 31) - 1) return fail(ctx, RT_ERR_INVALID_ARGUMENT, "image too large");
-                cur.push_back(PartDev{j, pass, (int)used, (int)npix, np, {0, 0, 0}});
+                cur.push_back(PartDev{j, pass, (int)used, (int)npix, np, st->width, {0, 0}});
                 used += np * npix;
                 pass += np;
             }
