@@ -1,19 +1,20 @@
 // render.hip — wavefront path tracer for gfx950 and the C ABI (include/rt3d.h).
 //
-// One camera sample = one path slot for the lifetime of a chunk.  A chunk is
-// K whole sample passes over the image (path p = s_local * W*H + pixel), so
-// the per-pixel film sum is taken in sample order exactly like the
-// reference's `cumulativeColor += sample` (Renderer.cs:668-672).  Each bounce
-// runs as its own stage:
+// A pool of path slots runs the camera samples of a window (whole sample
+// passes of the image).  A slot whose path ends restarts on the window's next
+// sample; each sample's result is stored under its number, and k_accum sums
+// a pixel's samples in order, as the reference's `cumulativeColor += sample`
+// does (Renderer.cs:668-672).  Each bounce runs as its own stages:
 //   k_raygen   camera rays, Sobol dims 0-1 (+ lens)      Renderer.cs:630-653
-//   k_trace    closest hit of the active queue          Renderer.cs:1609-1644
-//   k_shade    medium free flight, emission with MIS, NEE light samples
-//              (shadow rays queued), BSDF sample, Russian roulette, next
-//              ray; survivors are compacted into the next queue with a
-//              wave-aggregated atomic                    Renderer.cs:1008-1383, 1700-1782
+//   k_trace    closest hits of the pending slots         Renderer.cs:1609-1644
+//   k_shade    NEE phase: medium free flight, emission with MIS, light
+//              samples; bounce phase: their BSDF values, shadow rays
+//              queued, BSDF sample, roulette, next ray    Renderer.cs:1008-1383, 1700-1782
+//   k_gather   photon-caustics estimate                   Renderer.cs:1449-1508
 //   k_shadow   transparent shadow walk of the queued shadow rays
 //                                                        ShadowRay.cs:59-158
-//   k_finalize per-pixel clamp + film accumulation       Renderer.cs:668-721
+//   k_scan, k_retire   results of the ended paths, restarts
+//                                                        Renderer.cs:658-672
 //
 // The recursion's radiance sum L = Le0 + Ld0 + clampInd(att0 · L1) is
 // carried forward with two accumulators per path (primary-vertex terms and
@@ -197,43 +198,42 @@ struct ManyJobs {
     }
 };
 
-// counters[] (device-resident loop state):
-//   per iteration (cleared by k_iter_begin): paths active in the next
-//   iteration, shadow-queue size (ungrouped form), retired paths, gather
-//   requests, one size per light-sample segment of the grouped shadow queue;
-//   per window: next window sample to start, window size, paths active in
-//   the current iteration; per render: stack-overflow flag.
-constexpr int kCntNext = 0, kCntShadow = 1, kCntRetire = 2, kCntGather = 3, kCntSeg = 4, kMaxSeg = 32,
-              kCntClear = 40, kCntSid = 40, kCntWs = 41, kCntActive = 42, kCntSidSnap = 43, kCntWindow = 48,
-              kCntPend = 52, kCntOverflow = 63;
+// counters[] (device-resident loop state), per window: next window sample to
+// start, window size, first window sample of this iteration's restarts, and
+// for the host (kCntPend..+2, written by k_scan): paths pending in the next
+// iteration, the stack-overflow flag, and whether the window's samples are
+// all issued; per render: stack-overflow flag.
+constexpr int kCntSid = 0, kCntWs = 1, kCntSidBase = 2, kCntPend = 4, kCntWindow = 16, kCntOverflow = 63;
+constexpr int kMaxSeg = 32;     // light samples per vertex the grouped shadow mask holds
 // tcount[] (64-bit): traversal tests (trace node/tri/other, shadow node/tri/other), closest-hit segments, shadow rays
 constexpr int kTcRays = 6, kTcShadowRays = 7;
 // any-hit (4-wide BVH) traversal work of the shadow kernel: node fetches, triangle/quad/plane tests, sphere tests
 constexpr int kTcAnyNode = 8, kTcAnyTri = 9, kTcAnyOther = 10;
-// per-wave count arrays (wc): continuing paths, retired paths, gather
-// requests, shadow rays (ungrouped form), then one per light-sample segment
-constexpr int kWcNext = 0, kWcRetire = 1, kWcGather = 2, kWcShadow = 3, kWcSeg = 4;
-constexpr int kCntSidBase = 44;   // first window sample of this iteration's restarts
-// kCntPend..+2 (written by k_batch_end for the host): paths pending in the next
-// iteration, the stack-overflow flag, and whether the window's samples are all issued
+// per-chunk count arrays (wc): continuing paths, retired paths
+constexpr int kWcNext = 0, kWcRetire = 1, kWcRows = 2;
+// Queue sizes (seg), one 128-byte line each: the shadow queue has a segment
+// per light sample (ungrouped form: one) and per stripe of the workgroups
+// that fill it (at most 64 in all, a lane each), so the chunks' atomics
+// spread over that many lines; stripe x of segment j is size j * stripes + x.
+// The gather queue is the last.
+constexpr int kSegStride = 32, kSegGather = 64, kSegs = 65, kStripes = 8;
+RT_HD int shadow_stripes(int maxs) { return maxs <= 8 || maxs > kMaxSeg ? kStripes : maxs <= 16 ? 4 : 2; }
 constexpr int kIterBatch = 4;   // bounce iterations enqueued between host checks
-// kSlotBounce: shaded by the NEE phase of a split shade, waiting for its
-// BSDF bounce (k_shade<..., kPhBounce>) in the same iteration
-enum : int32_t { kSlotIdle = 0, kSlotActive = 1, kSlotRetired = 2, kSlotBounce = 3 };
+// Slot states.  Between iterations: idle, active (continues), fresh (a camera
+// ray to trace) or retired (k_retire takes it; samples of depth-0 jobs start
+// there).  k_trace leaves hit (fresh or not) or miss, the NEE phase hands
+// scattering vertices to the bounce phase as kSlotBounceD (Disney) or
+// kSlotBounceO (the other materials).
+enum : uint8_t {
+    kSlotIdle = 0, kSlotActive = 1, kSlotRetired = 2, kSlotFresh = 3, kSlotHit = 4, kSlotHitFresh = 5, kSlotMiss = 6,
+    kSlotBounceD = 7, kSlotBounceO = 8
+};
 // Shading phases: the whole vertex in one kernel (kept for the adjoint's
 // replay pass), or split in two launches — medium, emission, NEE and the
 // caustic gather request first, then the BSDF sample, roulette and next ray
 // of surface vertices — so that neither kernel holds both the light-sample
 // and the BSDF-sample state.
 enum : int { kPhAll = 0, kPhNee = 1, kPhBounce = 2 };
-
-// Shadow queue view: segment j holds the shadow rays of light sample j
-// (in light-list order) at q_sh[j*stride ...]; pre[] is the prefix of the
-// segment sizes, so launch index i maps to segment j with pre[j] <= i < pre[j+1].
-struct ShQ {
-    int nseg, stride;
-    int pre[kMaxSeg + 1];
-};
 
 struct PathBufs {
     float4 *o, *d, *thr, *wt, *w0, *a0, *ai, *ab;
@@ -243,13 +243,16 @@ struct PathBufs {
     int4* hit_xf;               // wrapper chain of the hit (scenes with an object hierarchy)
     float4 *av0, *av1, *av2, *av3, *av4;   // AOV probe
     float4 *sh_o, *sh_d, *sh_c, *sh_r;     // shadow records, record k of slot p at k*N + p (N × maxs)
-    int32_t* state;             // per slot: kSlotIdle, kSlotActive (to trace), kSlotRetired
-    int32_t* gflag;             // per slot: a caustic gather request was queued this iteration
+    uint8_t* state;             // per slot: kSlot* above
+    uint8_t* gflag;             // per slot: a caustic gather request was queued this iteration
+    int32_t* wc;                // per-chunk counts, kWcRows rows; the retire row is scanned in place
+    int nw;                     // row stride of wc: chunks rounded up to a multiple of 4
+    int wide, chunk;            // slots per chunk of the four-wave and the one-wave kernels
+    int32_t* q_sh;              // shadow queue: record indices, segment j stripe x from q_seg * (j * stripes + x)
+    int q_seg;                  // entries a stripe of a segment can hold
     int32_t* q_g;               // gather queue: slots with a request
-    int32_t* wc;                // per-wave counts, kWc* arrays of ceil(N/64) entries, scanned in place
-    int nw;                     // row stride of wc: ceil(N/64) rounded up to a multiple of 4
-    int32_t* smask;             // per slot: light samples with a pending shadow ray (grouped form)
-    int32_t* q_sh;              // shadow queue: shadow record indices
+    int32_t* seg;               // queue sizes, size j at j * kSegStride
+    int32_t* smask;             // per slot: light samples with a pending shadow ray (their number if maxs > kMaxSeg)
     int32_t* sid;               // sample of the window each path slot is tracing
     int32_t *job, *pix, *pass;  // its job (batch), pixel index and sample pass
     const struct PartDev* parts;   // window parts (job, first pass, window offset)
@@ -314,18 +317,117 @@ __device__ __forceinline__ int pf_cat(int32_t f) { return (f >> kPfCatShift) & 3
 __device__ __forceinline__ int pf_pend(int32_t f) { return (f >> kPfPendShift) & 0xff; }
 
 // XCD-aware block order: gfx950 dispatches consecutive workgroups round-robin
-// over its 8 XCDs; renumber so each XCD walks runs of kXcdRun consecutive
+// over its 8 XCDs; renumber so each XCD walks runs of `run` consecutive
 // blocks (neighbouring rays share BVH nodes in that XCD's L2) while the eight
-// stay side by side in the queue, so sky and object parts of the image load
-// them evenly (one eighth of the pool per XCD ran that frame in 349 ms).
-constexpr uint32_t kXcdRun = 32;
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb) {
-    const uint32_t whole = nb / (8u * kXcdRun) * (8u * kXcdRun);
+// stay side by side in the pool, so sky and object parts of the image load
+// them evenly (one eighth of the pool per XCD ran the 1080p frame in 349
+// instead of 298 ms).  Runs of 2048 slots.
+constexpr uint32_t kXcdSlots = 2048;
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb, uint32_t run) {
+    const uint32_t whole = nb / (8u * run) * (8u * run);
     if (b >= whole) return b;   // the last, partial round keeps its order
     const uint32_t x = b % 8u, i = b / 8u;
-    return (i / kXcdRun * 8u + x) * kXcdRun + i % kXcdRun;
+    return (i / run * 8u + x) * run + i % run;
 }
-__device__ __forceinline__ uint32_t xcd_block() { return xcd_remap(blockIdx.x, gridDim.x); }
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_remap(blockIdx.x, gridDim.x, kXcdSlots / kBlock); }
+
+// ── chunks: the pool kernels' unit of work ───────────────────────────────
+// A workgroup of WAVES waves owns a chunk of consecutive slots, lists the
+// ones its stage works on in LDS, class by class, and its waves take them 64
+// at a time: full waves whatever share of the slots is live, camera rays
+// beside camera rays, and no queue in memory.  k_trace runs four waves on up
+// to kChunkMax slots (a ray's cost varies: the waves take batches as they
+// get free); the bounce phase and k_retire run one wave on up to kChunkOne
+// slots (their vertices cost about the same, and a lone wave waits for
+// nobody); the NEE phase runs four waves in pools of kNeeWide slots or more
+// (3.03 against 3.17 ms a launch at 33.5 M slots), one in smaller ones (40
+// against 51 us at 2 M).  Chunks are as large as leaves a few rounds of
+// workgroups: at 1 M slots 192 slots a wave shade a bounce phase in 57 us, 64
+// in 68; at 2 M 256 in 150, 448 in 187.
+constexpr int kWaves = 4, kWg = kWaves * kBlock;
+constexpr int kChunkMax = 1024, kChunkOne = 512, kNeeWide = 1 << 22;
+inline int chunk_wide(int64_t n) {
+    const int64_t c = n / 8192 / kWg * kWg;
+    return (int)(c < kWg ? kWg : c > kChunkMax ? kChunkMax : c);
+}
+inline int chunk_one(int64_t n) {
+    const int64_t c = std::max(std::min<int64_t>(n / 4096, 256), n / 32768) / kBlock * kBlock;
+    return (int)(c < kBlock ? kBlock : c > kChunkOne ? kChunkOne : c);
+}
+__device__ __forceinline__ int chunk_base(int chunk) {
+    return (int)xcd_remap(blockIdx.x, gridDim.x, kXcdSlots / (uint32_t)chunk) * chunk;
+}
+
+// The chunk's slots by class of their state: cls(state) = 0 or 1 lists the
+// slot, 2 and 3 only count it, < 0 skips it.
+struct ChunkList {
+    int n0, n1, c2, c3;
+    const uint16_t* q;          // class 0 from the front, class 1 from the back
+    int* next;                  // next batch of 64 to take
+    int size;
+    __device__ __forceinline__ int total() const { return n0 + n1; }
+    __device__ __forceinline__ int at(int t) const { return t < n0 ? q[t] : q[size - 1 - (t - n0)]; }
+    // the wave's next batch: first list index (>= total(): none left)
+    __device__ __forceinline__ int take() const {
+        int t = 0;
+        if (__lane_id() == 0) t = atomicAdd(next, kBlock);
+        return __builtin_amdgcn_readfirstlane(t);
+    }
+};
+template <int WAVES, int MAX>
+struct ChunkLds {
+    uint16_t q[MAX];
+    int start[kMaxSeg];         // queue_shadows
+    int cnt[4][WAVES];
+    int next;
+};
+template <int WAVES, int MAX, class F>
+__device__ __forceinline__ ChunkList chunk_list(const uint8_t* __restrict__ state, int base, int n, int chunk,
+                                                ChunkLds<WAVES, MAX>& l, F&& cls) {
+    constexpr int kRows = MAX / (WAVES * kBlock);   // 64-slot rows per wave
+    const int lane = (int)__lane_id(), wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kBlock);
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    const int per = chunk / WAVES, r0 = wid * per;
+    int c[kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; k++) {
+        const int r = k * kBlock + lane, p = base + r0 + r;
+        c[k] = r < per && p < n ? cls(state[p]) : -1;
+    }
+    int m[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < kRows; k++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) m[j] += __popcll(__ballot(c[k] == j));
+    if (lane == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) l.cnt[j][wid] = m[j];
+        if (wid == 0) l.next = 0;
+    }
+    __syncthreads();
+    int tot[4] = {0, 0, 0, 0}, f = 0, g = 0;   // f, g: classes 0 and 1 of the waves before this one
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        if (w == wid) {
+            f = tot[0];
+            g = tot[1];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) tot[j] += l.cnt[j][w];
+    }
+#pragma unroll
+    for (int k = 0; k < kRows; k++) {
+        const int r = r0 + k * kBlock + lane;
+        const unsigned long long b0 = __ballot(c[k] == 0), b1 = __ballot(c[k] == 1);
+        if (c[k] == 0) l.q[f + __popcll(b0 & lt)] = (uint16_t)r;
+        if (c[k] == 1) l.q[chunk - 1 - g - __popcll(b1 & lt)] = (uint16_t)r;
+        f += __popcll(b0);
+        g += __popcll(b1);
+    }
+    __syncthreads();
+    auto u = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    return ChunkList{u(tot[0]), u(tot[1]), u(tot[2]), u(tot[3]), l.q, &l.next, chunk};
+}
 
 
 // ── surface reconstruction from an entry (primitive Hit bodies) ─────────
@@ -965,7 +1067,7 @@ __device__ __forceinline__ void resolve_sample(const PathBufs& P, int sid, int& 
 
 // Starts the camera path of window sample `sid` (pixel `pix`, sample pass
 // `pass` of job `job`) in slot p.
-__device__ __forceinline__ void init_path(const DevScene& S, const RParams& R, PathBufs& P, int p, int sid, int job,
+__device__ __forceinline__ void init_path(const DevScene& S, const RParams& R, const PathBufs& P, int p, int sid, int job,
                                           int pix, int pass) {
     int i = pix % R.W, j = pix / R.W;
     pass += R.soff;   // the sample's global index (Sobol index, half parity)
@@ -996,57 +1098,25 @@ __device__ __forceinline__ void init_path(const DevScene& S, const RParams& R, P
 // Initial fill of the path pool: slot p < n traces window sample p; the
 // rest of the pool stays idle.
 template <class JOBS>
-__global__ void __launch_bounds__(kBlock) k_raygen(JOBS jobs, PathBufs P, int n, int ws) {
+__global__ void __launch_bounds__(kBlock) k_raygen(JOBS jobs, PathBufs P, int n, int ws, int traced) {
     int p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= P.n) return;
-    int st = kSlotIdle;
+    uint8_t st = kSlotIdle;
     if (p < n) {
         int job, pix, pass;
         resolve_sample(P, p, job, pix, pass);
         const RParams& R = jobs.params(job);
         init_path(jobs.scene(job), R, P, p, p, job, pix, pass);
-        st = R.max_depth > 0 ? kSlotActive : kSlotRetired;
+        st = R.max_depth > 0 ? kSlotFresh : kSlotRetired;
     }
     P.state[p] = st;
+    P.smask[p] = 0;
+    if (P.q_g) P.gflag[p] = 0;
     if (p == 0) {
-        P.counters[kCntNext] = n;
         P.counters[kCntSid] = n;
-        P.counters[kCntSidSnap] = n;
         P.counters[kCntWs] = ws;
-    }
-}
-
-// Start of one bounce iteration: count the paths pending in it (paths that
-// continued from the previous iteration + slots the previous k_retire
-// restarted, derived from the window's sample counter), add the previous
-// iteration's traced and shadow segments to the statistics, clear the
-// per-iteration counters.  One wave.
-__global__ void __launch_bounds__(kBlock) k_iter_begin(PathBufs P, int traced) {
-    if (threadIdx.x == 0) {
-        const int sid = P.counters[kCntSid], snap = P.counters[kCntSidSnap], ws = P.counters[kCntWs];
-        const int started = min(sid - snap, max(0, ws - snap));
-        int active = P.counters[kCntNext] + started;
-        P.counters[kCntSidSnap] = sid;
-        long long sh = P.counters[kCntShadow];
-        for (int j = 0; j < kMaxSeg; j++) sh += P.counters[kCntSeg + j];
-        P.counters[kCntActive] = active;
-        if (traced && active > 0) P.tcount[kTcRays] += (unsigned long long)active;
-        if (sh > 0) P.tcount[kTcShadowRays] += (unsigned long long)sh;
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < kCntClear; k += kBlock) P.counters[k] = 0;
-}
-
-// End of a batch of iterations: the paths pending in the next iteration
-// (k_iter_begin's count, without its side effects), the overflow flag and
-// whether every sample of the window has been issued, for one host copy.
-__global__ void __launch_bounds__(kBlock) k_batch_end(PathBufs P) {
-    if (threadIdx.x == 0) {
-        const int sid = P.counters[kCntSid], snap = P.counters[kCntSidSnap], ws = P.counters[kCntWs];
-        const int started = min(sid - snap, max(0, ws - snap));
-        P.counters[kCntPend] = P.counters[kCntNext] + started;
-        P.counters[kCntPend + 1] = P.counters[kCntOverflow];
-        P.counters[kCntPend + 2] = sid >= ws ? 1 : 0;
+        for (int j = 0; j < kSegs; j++) P.seg[j * kSegStride] = 0;
+        if (traced) P.tcount[kTcRays] += (unsigned long long)n;
     }
 }
 
@@ -1056,46 +1126,54 @@ __global__ void __launch_bounds__(kBlock) k_batch_end(PathBufs P) {
 // faster than the 7-wave build), batches of flat scenes for 7; the
 // wrapper-entry traversal takes the registers it needs (3-4 waves).
 template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
-__global__ void __launch_bounds__(kBlock, XF ? 1 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
+__global__ void __launch_bounds__(kWg, XF ? 1 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
     k_trace(JOBS jobs, PathBufs P) {
-    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
+    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kWg];
+    __shared__ ChunkLds<kWaves, kChunkMax> lds;
     uint2 priv_stk[PRIV ? SD : 1];
     uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
-    constexpr int STRIDE = PRIV ? 1 : kBlock;
+    constexpr int STRIDE = PRIV ? 1 : kWg;
     TravCount tc{0u, 0u, 0u};
-    const int p = xcd_block() * kBlock + threadIdx.x;
-    if (p >= P.n || P.state[p] != kSlotActive) {
-        if (COUNT) flush_counts(P.tcount, tc);
-        return;
-    }
-    jobs.run_lane(true, jobs.job_of(P.job, p), [&](const DevScene& S, const RParams&) {
-        float4 o4 = P.o[p], d4 = P.d[p];
-        f3 o = f3of(o4), d = f3of(d4);
-        bool camera = pf_cat(__float_as_int(d4.w)) == 0;
-        HitOut h;
-        bool moved = false;
-        for (int skip = 0;;) {
-            h = trace_closest<SD, STRIDE, COUNT, false, XF>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d,
-                                                            kEps, kInfinity, stk, (uint32_t*)&P.counters[kCntOverflow],
-                                                            tc, S.xf);
-            if (h.entry < 0 || !camera) break;
-            if (XF) {
-                if (!hit_cam_invisible(S, h.entry, h.chain)) break;
-                f3 lo, ld;
-                o = offset_origin(make_surf_w(S, h.entry, h.chain, o, d, h.t, h.u, h.v, lo, ld).p, d);
-            } else {
-                int32_t fl = tag_of(S.entries[h.entry].a) >> 8;
-                if (!(fl & kEntryCamInvisible)) break;
-                o = offset_origin(o + h.t * d, d);
-            }
-            moved = true;
-            if (++skip >= 8) break;
-        }
-        if (moved) P.o[p] = make_float4(o.x, o.y, o.z, o4.w);
-        P.hit_e[p] = h.entry;
-        P.hit_tuv[p] = make_float4(h.t, h.u, h.v, 0.0f);
-        if (XF) P.hit_xf[p] = h.chain;
+    const int base = chunk_base(P.wide);
+    // camera rays first, continuing paths after them
+    const ChunkList L = chunk_list(P.state, base, P.n, P.wide, lds, [](uint8_t st) {
+        return st == kSlotFresh ? 0 : st == kSlotActive ? 1 : -1;
     });
+    for (int t0 = L.take(); t0 < L.total(); t0 = L.take()) {
+        const int t = t0 + (int)__lane_id();
+        if (t >= L.total()) break;
+        const int p = base + L.at(t);
+        const bool fresh = t < L.n0;
+        jobs.run_lane(true, jobs.job_of(P.job, p), [&](const DevScene& S, const RParams&) {
+            float4 o4 = P.o[p], d4 = P.d[p];
+            f3 o = f3of(o4), d = f3of(d4);
+            bool camera = pf_cat(__float_as_int(d4.w)) == 0;
+            HitOut h;
+            bool moved = false;
+            for (int skip = 0;;) {
+                h = trace_closest<SD, STRIDE, COUNT, false, XF>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o,
+                                                                d, kEps, kInfinity, stk,
+                                                                (uint32_t*)&P.counters[kCntOverflow], tc, S.xf);
+                if (h.entry < 0 || !camera) break;
+                if (XF) {
+                    if (!hit_cam_invisible(S, h.entry, h.chain)) break;
+                    f3 lo, ld;
+                    o = offset_origin(make_surf_w(S, h.entry, h.chain, o, d, h.t, h.u, h.v, lo, ld).p, d);
+                } else {
+                    int32_t fl = tag_of(S.entries[h.entry].a) >> 8;
+                    if (!(fl & kEntryCamInvisible)) break;
+                    o = offset_origin(o + h.t * d, d);
+                }
+                moved = true;
+                if (++skip >= 8) break;
+            }
+            if (moved) P.o[p] = make_float4(o.x, o.y, o.z, o4.w);
+            P.hit_e[p] = h.entry;
+            P.hit_tuv[p] = make_float4(h.t, h.u, h.v, 0.0f);
+            P.state[p] = h.entry < 0 ? kSlotMiss : fresh ? kSlotHitFresh : kSlotHit;
+            if (XF) P.hit_xf[p] = h.chain;
+        });
+    }
     if (COUNT) flush_counts(P.tcount, tc);
 }
 
@@ -1142,7 +1220,7 @@ __global__ void __launch_bounds__(kBlock) k_fp(JOBS jobs, PathBufs P) {
     uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
     constexpr int STRIDE = PRIV ? 1 : kBlock;
     const int p = xcd_block() * kBlock + threadIdx.x;
-    if (p >= P.n || P.state[p] != kSlotActive) return;
+    if (p >= P.n || (P.state[p] != kSlotHit && P.state[p] != kSlotHitFresh)) return;
     jobs.run(true, jobs.job_of(P.job, p), [&](const DevScene& S, const RParams& R) {
         float4 fp = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const int he = P.hit_e[p];
@@ -1188,7 +1266,7 @@ __global__ void __launch_bounds__(kBlock) k_fp(JOBS jobs, PathBufs P) {
     });
 }
 
-__device__ __forceinline__ void add_target(PathBufs& P, int p, bool ind, f3 c) {
+__device__ __forceinline__ void add_target(const PathBufs& P, int p, bool ind, f3 c) {
     float4* acc = ind ? P.ai : P.a0;
     float4 a = acc[p];
     acc[p] = make_float4(a.x + c.x, a.y + c.y, a.z + c.z, a.w);
@@ -1196,7 +1274,7 @@ __device__ __forceinline__ void add_target(PathBufs& P, int p, bool ind, f3 c) {
 
 // Adds the transmittance-weighted shadow contributions of the path's last
 // vertex to its accumulator, in light/sample order.
-__device__ __forceinline__ int32_t fold_shadows(PathBufs& P, const RParams& R, int p, int32_t flags) {
+__device__ __forceinline__ int32_t fold_shadows(const PathBufs& P, const RParams& R, int p, int32_t flags) {
     int pend = pf_pend(flags);
     if (pend == 0) return flags;
     f3 s = splat(0.0f);
@@ -1228,19 +1306,40 @@ __device__ __forceinline__ int32_t fold_shadows(PathBufs& P, const RParams& R, i
 // RND: the PRNG sampler mode, fixed per kernel so the Sobol kernels carry no
 // code of the other mode.  UL: every job of the launch samples all lights
 // (no light pick), so the NEE light loop runs over a wave-uniform index.
-template <class JOBS, int WPE, bool ADJ = false, int PH = kPhAll, bool TF = true, bool RND = false, bool UL = false>
-__global__ void __launch_bounds__(kBlock, WPE) k_shade(JOBS jobs, PathBufs P, int maxs) {
+// The kernel's arguments as they lie in the argument segment.  Read through
+// a pointer the compiler cannot see through, so that a batch loads the fields
+// it uses with scalar loads where it uses them: hoisted out of the batch
+// loop, the hundred-odd pointers and parameters would be spilled.
+template <class JOBS>
+struct ShadeArgs {
+    JOBS jobs;
+    PathBufs P;
+    int maxs;
+};
+template <class JOBS>
+__device__ __forceinline__ const ShadeArgs<JOBS>& shade_args() {
+    typedef const __attribute__((address_space(4))) ShadeArgs<JOBS> A;
+    A* a = (A*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return *(const ShadeArgs<JOBS>*)a;
+}
+
+struct ShadeOut {
+    int n_shadow;
+    uint32_t smask;
+    bool cont, bounce, disney_vtx, gather;
+};
+template <class JOBS, bool ADJ, int PH, bool TF, bool RND, bool UL>
+__device__ __forceinline__ ShadeOut shade_slot(const JOBS& jobs, const PathBufs& P, int maxs, int p, bool active) {
     static_assert(!ADJ || PH == kPhAll, "the adjoint replay shades whole vertices");
     constexpr bool kFront = PH != kPhBounce;    // medium, emission, NEE, gather
     constexpr bool kBack = PH != kPhNee;        // BSDF bounce
-    const int p = xcd_block() * kBlock + threadIdx.x;
-    const int st_in = p < P.n ? P.state[p] : kSlotIdle;
-    const bool active = st_in == (PH == kPhBounce ? kSlotBounce : kSlotActive);
     const int job = active ? jobs.job_of(P.job, p) : 0;
     int n_shadow = 0;
     uint32_t smask = 0;   // bit j: light sample j produced a shadow ray
     bool cont = false;
     bool bounce = false;  // kPhNee: the vertex waits for its BSDF bounce
+    bool disney_vtx = false;
     bool gather = false;  // a caustic gather request was queued
     // per-lane shadow records are written straight into the path's slots
     jobs.run_lane(active, job, [&](const DevScene& S, const RParams& R) {
@@ -1566,6 +1665,7 @@ __global__ void __launch_bounds__(kBlock, WPE) k_shade(JOBS jobs, PathBufs P, in
                 }
                 // the NEE phase hands scattering vertices to the bounce phase
                 bounce = scatters;
+                disney_vtx = kind == RT_MAT_DISNEY;
                 if (bounce) {
                     const f3 ts = thr * mb;
                     P.thr[p] = make_float4(ts.x, ts.y, ts.z, __int_as_float(depth));
@@ -1915,100 +2015,218 @@ __global__ void __launch_bounds__(kBlock, WPE) k_shade(JOBS jobs, PathBufs P, in
             }
         }
     });
-    // slot state, per-slot outputs and this wave's counts (no atomics: the
-    // queues are laid out by k_wave_scan + k_compact from the counts)
-    const bool retire = active && !cont && !bounce;
-    if (p < P.n) {
-        if (PH == kPhBounce) {
-            if (active) {
-                P.state[p] = cont ? kSlotActive : kSlotRetired;
-                P.smask[p] = maxs <= kMaxSeg ? (int32_t)smask : n_shadow;
-            }
-        } else {
-            if (retire) P.state[p] = kSlotRetired;
-            else if (bounce) P.state[p] = kSlotBounce;
-            P.smask[p] = maxs <= kMaxSeg ? (int32_t)smask : n_shadow;
-            P.gflag[p] = gather ? 1 : 0;
-        }
+    return ShadeOut{n_shadow, smask, cont, bounce, disney_vtx, gather};
+}
+
+// Queues the chunk's shadow rays, all workgroup: the slots' masks (every
+// slot's: the NEE phase of a medium vertex may have left some) are read back,
+// counted per light sample and 64-slot row, one atomic per light sample takes
+// the chunk's range of its segment, and the records follow in slot order, so
+// a wave of k_shadow traces neighbouring paths' rays toward one light.  The
+// list memory is free by now.
+template <int WAVES, int MAX>
+__device__ __forceinline__ void queue_shadows(const PathBufs& P, int maxs, int base, ChunkLds<WAVES, MAX>& l) {
+    constexpr int kRows = MAX / (WAVES * kBlock);
+    const int lane = (int)__lane_id(), wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kBlock);
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    const int rows = P.chunk / (WAVES * kBlock), row0 = wid * rows;       // this wave's rows of the chunk
+    const bool grouped = maxs <= kMaxSeg;
+    uint32_t m[kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; k++) {
+        const int p = base + (row0 + k) * kBlock + lane;
+        m[k] = k < rows && p < P.n ? (uint32_t)P.smask[p] : 0u;
     }
-    const int w = p >> 6;
-    if (PH != kPhNee) {
-        // continuing and retired paths: retired this iteration, plus slots
-        // restarted as already-retired (samples of depth-0 jobs), which
-        // k_retire finishes as well; the bounce phase also counts the
-        // vertices the NEE phase ended or continued (medium scattering)
-        const bool is_cont = PH == kPhBounce ? (active ? cont : st_in == kSlotActive) : cont;
-        const bool is_ret = PH == kPhBounce ? (active ? !cont : st_in == kSlotRetired) : (retire || st_in == kSlotRetired);
-        const int n_cont = __popcll(__ballot(is_cont)), n_ret = __popcll(__ballot(is_ret));
-        // shadow rays of every slot: the bounce phase's own vertices after the
-        // BSDF evaluation, the others as the NEE phase left them
-        uint32_t sm = smask;
-        int nsh = n_shadow;
-        if (PH == kPhBounce && !active) {
-            const int32_t m = p < P.n ? P.smask[p] : 0;
-            sm = maxs <= kMaxSeg ? (uint32_t)m : 0u;
-            nsh = maxs <= kMaxSeg ? 0 : m;
+    uint32_t any = 0;
+#pragma unroll
+    for (int k = 0; k < kRows; k++) any |= m[k];
+    static_assert(WAVES == 1, "one wave decides for the chunk");
+    if (__ballot(any != 0u) == 0ull) return;
+    const int stripes = shadow_stripes(maxs), x = (int)(blockIdx.x % (unsigned)stripes);
+    if (grouped) {
+        // counts of (light sample j, row) at cnt[j * rows of the chunk + row]
+        static_assert(MAX / kBlock * kMaxSeg <= MAX, "counts fit the list memory");
+        uint16_t* cnt = l.q;
+        int* start = l.start;
+        const int all = rows * WAVES;
+        for (int j = 0; j < maxs; j++)
+#pragma unroll
+            for (int k = 0; k < kRows; k++)
+                if (k < rows) {
+                    const int c = __popcll(__ballot((m[k] >> j) & 1u));
+                    if (lane == 0) cnt[j * all + row0 + k] = (uint16_t)c;
+                }
+        __syncthreads();
+        if ((int)threadIdx.x < maxs) {
+            int t = 0;
+            for (int r = 0; r < all; r++) {
+                const int c = cnt[threadIdx.x * all + r];
+                cnt[threadIdx.x * all + r] = (uint16_t)t;
+                t += c;
+            }
+            start[threadIdx.x] = t > 0 ? atomicAdd(&P.seg[(threadIdx.x * stripes + x) * kSegStride], t) : 0;
         }
-        for (int off = 32; off > 0; off >>= 1) nsh += __shfl_xor(nsh, off, 64);
+        __syncthreads();
+        for (int j = 0; j < maxs; j++) {
+            int32_t* q = P.q_sh + (int64_t)P.q_seg * (j * stripes + x) + start[j];
+#pragma unroll
+            for (int k = 0; k < kRows; k++)
+                if (k < rows) {
+                    const bool h = (m[k] >> j) & 1u;
+                    const unsigned long long b = __ballot(h);
+                    if (h)
+                        q[cnt[j * all + row0 + k] + __popcll(b & lt)] =
+                            (int32_t)((int64_t)j * P.n + base + (row0 + k) * kBlock + lane);
+                }
+        }
+    } else {
+        // the slots' records one after the other
+        int incl[kRows], t = 0;
+#pragma unroll
+        for (int k = 0; k < kRows; k++) {
+            int c = (int)m[k];
+            for (int off = 1; off < 64; off <<= 1) {
+                const int y = __shfl_up(c, off, 64);
+                if (lane >= off) c += y;
+            }
+            incl[k] = t + c;
+            t += __shfl(c, 63, 64);
+        }
+        int w0 = 0;
+        if (lane == 0 && t > 0) w0 = atomicAdd(&P.seg[x * kSegStride], t);
+        w0 = __builtin_amdgcn_readfirstlane(w0);
+#pragma unroll
+        for (int k = 0; k < kRows; k++)
+            for (int i = 0; i < (int)m[k]; i++)
+                P.q_sh[(int64_t)P.q_seg * x + w0 + incl[k] - (int)m[k] + i] =
+                    (int32_t)((int64_t)i * P.n + base + (row0 + k) * kBlock + lane);
+    }
+}
+
+// Queues the chunk's caustic gather requests the same way.
+template <int WAVES, int MAX>
+__device__ __forceinline__ void queue_gathers(const PathBufs& P, int chunk, int base) {
+    constexpr int kRows = MAX / (WAVES * kBlock);
+    const int lane = (int)__lane_id(), wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kBlock);
+    const int per = chunk / WAVES, p0 = base + wid * per;
+    unsigned long long b[kRows];
+    int n = 0;
+#pragma unroll
+    for (int k = 0; k < kRows; k++) {
+        const int r = k * kBlock + lane, p = p0 + r;
+        b[k] = __ballot(r < per && p < P.n && P.gflag[p]);
+        n += __popcll(b[k]);
+    }
+    if (n == 0) return;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&P.seg[kSegGather * kSegStride], n);
+    at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int k = 0; k < kRows; k++) {
+        if ((b[k] >> lane) & 1ull)
+            P.q_g[at + __popcll(b[k] & ((1ull << lane) - 1ull))] = p0 + k * kBlock + lane;
+        at += __popcll(b[k]);
+    }
+}
+
+template <class JOBS, int WPE, bool ADJ = false, int PH = kPhAll, bool TF = true, bool RND = false, bool UL = false,
+          int WAVES = 1>
+__global__ void __launch_bounds__(WAVES * kBlock, WPE) k_shade(JOBS jobs, PathBufs P, int maxs) {
+    constexpr bool kFront = PH != kPhBounce, kBack = PH != kPhNee;
+    static_assert(WAVES == 1 || PH == kPhNee, "chunk counts are one wave's");
+    constexpr int kMax = WAVES == 1 ? kChunkOne : kChunkMax;
+    __shared__ ChunkLds<WAVES, kMax> lds;
+    const int chunk = WAVES == 1 ? P.chunk : P.wide;
+    const int base = chunk_base(chunk);
+    // NEE phase: hits, misses; bounce phase: Disney vertices, the other
+    // materials.  Slots that need no shading count as retired (2) or
+    // continuing (3).
+    const ChunkList L = chunk_list(P.state, base, P.n, chunk, lds, [](uint8_t st) {
+        if (kFront && (st == kSlotHitFresh || st == kSlotHit)) return 0;
+        if (kFront && st == kSlotMiss) return 1;
+        if (!kFront && st == kSlotBounceD) return 0;
+        if (!kFront && st == kSlotBounceO) return 1;
+        if (kBack && st == kSlotRetired) return 2;
+        if (!kFront && st == kSlotActive) return 3;
+        return -1;
+    });
+    int n_ret = L.c2, n_cont = L.c3;
+    for (int t0 = L.take(); t0 < L.total(); t0 = L.take()) {
+        const int t = t0 + (int)__lane_id();
+        const bool active = t < L.total();
+        const int p = base + (active ? L.at(t) : 0);
+        const ShadeArgs<JOBS>& A = shade_args<JOBS>();
+        const ShadeOut r = shade_slot<JOBS, ADJ, PH, TF, RND, UL>(A.jobs, A.P, maxs, p, active);
+        if (active) {
+            P.state[p] = r.bounce ? (r.disney_vtx ? kSlotBounceD : kSlotBounceO) : r.cont ? kSlotActive : kSlotRetired;
+            P.smask[p] = maxs <= kMaxSeg ? (int32_t)r.smask : r.n_shadow;
+            if (kFront && P.q_g) P.gflag[p] = r.gather ? 1 : 0;
+        }
+        n_cont += __popcll(__ballot(r.cont));
+        n_ret += __popcll(__ballot(active && !r.cont && !r.bounce));
+    }
+    __syncthreads();
+    if constexpr (kBack) {
+        // this chunk's counts (k_scan turns them into the restarts' sample numbers)
         if (threadIdx.x == 0) {
-            P.wc[kWcNext * P.nw + w] = n_cont;
-            P.wc[kWcRetire * P.nw + w] = n_ret;
-            P.wc[kWcShadow * P.nw + w] = maxs <= kMaxSeg ? 0 : nsh;
+            const int c = base / chunk;
+            P.wc[kWcNext * P.nw + c] = n_cont;
+            P.wc[kWcRetire * P.nw + c] = n_ret;
         }
-        if (maxs <= kMaxSeg)
-            for (int j = 0; j < maxs; j++) {
-                int c = __popcll(__ballot((sm >> j) & 1u));
-                if (threadIdx.x == 0) P.wc[(kWcSeg + j) * P.nw + w] = c;
-            }
-    }
-    if (PH != kPhBounce) {
-        const int n_g = __popcll(__ballot(gather));
-        if (threadIdx.x == 0) P.wc[kWcGather * P.nw + w] = n_g;
+        queue_shadows(P, maxs, base, lds);
+    } else if (P.q_g) {
+        queue_gathers<WAVES, kMax>(P, chunk, base);
     }
 }
 
-// Per-wave counts when no path is traced (depth-0 renders): every pending
-// slot is retired; the other count arrays are zero.
-__global__ void __launch_bounds__(kBlock) k_count_retired(PathBufs P, int narr) {
-    const int p = xcd_block() * kBlock + threadIdx.x;
-    const bool ret = p < P.n && P.state[p] == kSlotRetired;
-    const int n = __popcll(__ballot(ret));
-    if (threadIdx.x == 0)
-        for (int a = 0; a < narr; a++) P.wc[a * P.nw + (p >> 6)] = a == kWcRetire ? n : 0;
+// Per-chunk counts when no path is traced (depth-0 renders): every pending
+// slot is retired; the other counts are zero.
+__global__ void __launch_bounds__(kBlock) k_count_retired(PathBufs P) {
+    const int base = chunk_base(P.chunk);
+    int n = 0;
+    for (int r = threadIdx.x; r < P.chunk; r += kBlock) {
+        const int p = base + r;
+        n += p < P.n && P.state[p] == kSlotRetired;
+    }
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if (threadIdx.x == 0) {
+        const int c = base / P.chunk;
+        for (int a = 0; a < kWcRows; a++) P.wc[a * P.nw + c] = a == kWcRetire ? n : 0;
+    }
 }
 
-// Exclusive scan of one per-wave count array (block a scans array a) and
-// its total into the counters; the retire array also advances the window's
-// sample counter (the restarted slots take samples [sid, sid + total)).
-// Each thread owns kScanPer consecutive counts, read and written as int4
-// (a wave covers 8 KB of whole cache lines per round); a round scans
-// 1024 * kScanPer counts and the rounds carry the running total.
-constexpr int kScanPer = 32;
-__global__ void __launch_bounds__(1024) k_wave_scan(PathBufs P) {
-    __shared__ int32_t part[1024 / 64];
-    const int a = blockIdx.x;
-    int32_t* x = P.wc + (int64_t)a * P.nw;          // row stride P.nw: a multiple of 4
-    const int nwr = (P.n + kBlock - 1) / kBlock;    // counts written this iteration
+// End of an iteration, one workgroup: exclusive scan of the chunks' retired
+// counts (their restarted slots take window samples kCntSidBase + rank), the
+// window's sample counter, the statistics of the shadow rays just traced and
+// of the next iteration's segments, and the loop state the host polls.  Each
+// thread owns kScanPer consecutive chunks, read and written as int4.
+constexpr int kScanPer = 16;
+__global__ void __launch_bounds__(1024) k_scan(PathBufs P, int traced) {
+    __shared__ int32_t part[2][1024 / 64];
+    int32_t* x = P.wc + kWcRetire * P.nw;           // row stride P.nw: a multiple of 4
+    const int32_t* xn = P.wc + kWcNext * P.nw;
+    const int nch = (P.n + P.chunk - 1) / P.chunk;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     int carry = 0;
-    for (int r0 = 0; r0 < nwr; r0 += 1024 * kScanPer) {
+    int nnext = 0;
+    for (int r0 = 0; r0 < nch; r0 += 1024 * kScanPer) {
         const int b0 = r0 + (int)threadIdx.x * kScanPer;
         int v[kScanPer];
+        int next = 0;
 #pragma unroll
         for (int k = 0; k < kScanPer; k += 4) {
             const int i = b0 + k;
-            int4 q = make_int4(0, 0, 0, 0);
-            if (i + 3 < nwr) {
+            int4 q = make_int4(0, 0, 0, 0), qn = q;
+            if (i < nch) {   // rows are padded to whole int4s
                 q = *(const int4*)(x + i);
-            } else if (i < nwr) {
-                q.x = x[i];
-                if (i + 1 < nwr) q.y = x[i + 1];
-                if (i + 2 < nwr) q.z = x[i + 2];
+                qn = *(const int4*)(xn + i);
             }
+            const bool k1 = i + 1 < nch, k2 = i + 2 < nch, k3 = i + 3 < nch;
             v[k] = q.x;
-            v[k + 1] = q.y;
-            v[k + 2] = q.z;
-            v[k + 3] = q.w;
+            v[k + 1] = k1 ? q.y : 0;
+            v[k + 2] = k2 ? q.z : 0;
+            v[k + 3] = k3 ? q.w : 0;
+            next += qn.x + (k1 ? qn.y : 0) + (k2 ? qn.z : 0) + (k3 ? qn.w : 0);
         }
         int t = 0;
 #pragma unroll
@@ -2018,13 +2236,18 @@ __global__ void __launch_bounds__(1024) k_wave_scan(PathBufs P) {
             int y = __shfl_up(incl, off, 64);
             if (lane >= off) incl += y;
         }
-        if (lane == 63) part[wid] = incl;
+        for (int off = 32; off > 0; off >>= 1) next += __shfl_xor(next, off, 64);
+        if (lane == 63) {
+            part[0][wid] = incl;
+            part[1][wid] = next;
+        }
         __syncthreads();
         int wpre = 0, round = 0;
         for (int k = 0; k < 1024 / 64; k++) {
-            const int c = part[k];
+            const int c = part[0][k];
             wpre += k < wid ? c : 0;
             round += c;
+            nnext += part[1][k];
         }
         int run = carry + wpre + incl - t;
 #pragma unroll
@@ -2036,59 +2259,30 @@ __global__ void __launch_bounds__(1024) k_wave_scan(PathBufs P) {
             q.z = q.y + v[k + 1];
             q.w = q.z + v[k + 2];
             run = q.w + v[k + 3];
-            if (i + 3 < nwr) {
-                *(int4*)(x + i) = q;
-            } else if (i < nwr) {
-                x[i] = q.x;
-                if (i + 1 < nwr) x[i + 1] = q.y;
-                if (i + 2 < nwr) x[i + 2] = q.z;
-            }
+            if (i < nch) *(int4*)(x + i) = q;
         }
         carry += round;
         __syncthreads();   // part[] is rewritten by the next round
     }
     if (threadIdx.x == 0) {
-        const int total = carry;
-        const int slot = a == kWcNext ? kCntNext : a == kWcRetire ? kCntRetire : a == kWcGather ? kCntGather
-                       : a == kWcShadow ? kCntShadow : kCntSeg + (a - kWcSeg);
-        P.counters[slot] = total;
-        if (a == kWcRetire) {
-            P.counters[kCntSidBase] = P.counters[kCntSid];
-            P.counters[kCntSid] += total;
-        }
+        const int sid = P.counters[kCntSid], ws = P.counters[kCntWs];
+        const int started = min(carry, ws - sid);
+        const int pending = nnext + started;
+        P.counters[kCntSidBase] = sid;
+        P.counters[kCntSid] = sid + started;
+        P.counters[kCntPend] = pending;
+        P.counters[kCntPend + 1] = P.counters[kCntOverflow];
+        P.counters[kCntPend + 2] = sid + started >= ws ? 1 : 0;
+        if (traced && pending > 0) P.tcount[kTcRays] += (unsigned long long)pending;
     }
-}
-
-// Lays out the shadow queue (grouped by light sample, slot order within a
-// segment) and the gather queue from the scanned per-wave counts.
-__global__ void __launch_bounds__(kBlock) k_compact(PathBufs P, int maxs) {
-    const int p = xcd_block() * kBlock + threadIdx.x;
-    const bool ok = p < P.n;
-    const int w = p >> 6;
-    const unsigned long long lt = (1ull << (threadIdx.x & 63)) - 1ull;
-    const int st = ok ? P.state[p] : kSlotIdle;
-    const bool shaded = st != kSlotIdle;
-    const int m = shaded ? P.smask[p] : 0;
-    if (maxs <= kMaxSeg) {
-        for (int j = 0; j < maxs; j++) {
-            bool has = (m >> j) & 1;
-            unsigned long long b = __ballot(has);
-            if (has)
-                P.q_sh[(int64_t)j * P.n + P.wc[(kWcSeg + j) * P.nw + w] + __popcll(b & lt)] =
-                    (int32_t)((int64_t)j * P.n + p);
-        }
-    } else {
-        int incl = m;
-        for (int off = 1; off < 64; off <<= 1) {
-            int y = __shfl_up(incl, off, 64);
-            if ((int)(threadIdx.x & 63) >= off) incl += y;
-        }
-        int base = P.wc[kWcShadow * P.nw + w] + incl - m;
-        for (int k = 0; k < m; k++) P.q_sh[base + k] = (int32_t)((int64_t)k * P.n + p);
+    // the shadow rays traced this iteration; the next one queues from zero
+    if (wid == 0) {
+        long long t = P.seg[lane * kSegStride];
+        P.seg[lane * kSegStride] = 0;
+        if (lane == 0) P.seg[kSegGather * kSegStride] = 0;
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        if (lane == 0 && t > 0) P.tcount[kTcShadowRays] += (unsigned long long)t;
     }
-    const bool g = shaded && P.gflag[p];
-    unsigned long long gb = __ballot(g);
-    if (g) P.q_g[P.wc[kWcGather * P.nw + w] + __popcll(gb & lt)] = p;
 }
 
 }  // namespace rt
@@ -2100,21 +2294,12 @@ namespace rt {
 // :1520-1526): k nearest photons, cone filter k_f = 1 (normalisation 1/3),
 // adaptive radius, occupancy fade for sparse gathers.  Added to the target
 // accumulator of the path with the vertex weight.
-__global__ void __launch_bounds__(kBlock) k_gather(DevScene S, PathBufs P, DevPhotons M) {
-    const int count = P.counters[kCntGather];
-    const uint32_t nbk = (uint32_t)((count + kBlock - 1) / kBlock);
-    if (blockIdx.x >= nbk) return;
-    int i = xcd_remap(blockIdx.x, nbk) * kBlock + threadIdx.x;
-    if (i >= count) return;
-    const int slot = P.q_g[i];
+__device__ __forceinline__ void gather_slot(const DevScene& S, const PathBufs& P, const DevPhotons& M, int slot, float2* h) {
     float4 a = P.gq0[slot], b = P.gq1[slot], c = P.gq2[slot], w4 = P.gq3[slot];
     f3 o = f3of(a), d = f3of(b);
     Surf s = make_surf(S, __float_as_int(b.w), o, d, a.w, c.x, c.y);
     s.rel_eta = c.z;
     const int p = __float_as_int(c.w);
-    // the lane's heap of the k nearest photons, lane-interleaved in LDS
-    __shared__ float2 lds_h[kGatherK * kBlock];
-    float2* h = &lds_h[threadIdx.x];
     float radius;
     int n = photon_knn<kBlock>(M, s.p, h, radius);
     if (n == 0) return;
@@ -2149,44 +2334,21 @@ __global__ void __launch_bounds__(kBlock) k_gather(DevScene S, PathBufs P, DevPh
     add_target(P, p, __float_as_int(w4.w) != 0, sanitize(f3of(w4) * est));
 }
 
-// Transparent shadow walk (ShadowRay.Transmittance, ShadowRay.cs:59-158)
-template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
-__global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_shadow(JOBS jobs, PathBufs P, int maxs) {
-    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
-    uint2 priv_stk[PRIV ? SD : 1];
-    uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
-    constexpr int STRIDE = PRIV ? 1 : kBlock;
-    TravCount tc{0u, 0u, 0u};
-    // shadow queue view from the segment sizes (uniform over the grid)
-    const bool grouped = maxs <= kMaxSeg;
-    int total = grouped ? 0 : P.counters[kCntShadow];
-    if (grouped)
-        for (int j = 0; j < maxs; j++) total += P.counters[kCntSeg + j];
-    const uint32_t nb = (uint32_t)((total + kBlock - 1) / kBlock);
-    if (blockIdx.x >= nb) {
-        if (COUNT) flush_counts(P.tcount + 3, tc);
-        return;
-    }
-    int i = xcd_remap(blockIdx.x, nb) * kBlock + threadIdx.x;
-    if (i >= total) {
-        if (COUNT) flush_counts(P.tcount + 3, tc);
-        return;
-    }
-    int64_t qi = i;
-    int seg = 0;
-    if (grouped) {
-        int pre = 0;
-        for (;;) {
-            int c = P.counters[kCntSeg + seg];
-            if (i < pre + c || seg + 1 >= maxs) break;
-            pre += c;
-            seg++;
-        }
-        qi = (int64_t)seg * P.n + (i - pre);
-    }
-    int64_t sl = P.q_sh[qi];
-    // slot of the record: segment j holds light sample j's records at j*N + slot
-    const int slot = grouped ? (int)(sl - (int64_t)seg * P.n) : (int)(sl % P.n);
+__global__ void __launch_bounds__(kBlock) k_gather(DevScene S, PathBufs P, DevPhotons M) {
+    // the lane's heap of the k nearest photons, lane-interleaved
+    __shared__ float2 lds_h[kGatherK * kBlock];
+    const int count = P.seg[kSegGather * kSegStride];
+    const uint32_t nb = (uint32_t)((count + kBlock - 1) / kBlock);
+    if (blockIdx.x >= nb) return;
+    const int i = (int)xcd_remap(blockIdx.x, nb, kXcdSlots / kBlock) * kBlock + (int)threadIdx.x;
+    if (i < count) gather_slot(S, P, M, P.q_g[i], &lds_h[threadIdx.x]);
+}
+
+// Transparent shadow walk (ShadowRay.Transmittance, ShadowRay.cs:59-158) of
+// record sl of slot `slot`.
+template <class JOBS, int SD, int STRIDE, bool COUNT, bool XF>
+__device__ __forceinline__ void shadow_ray(const JOBS& jobs, const PathBufs& P, int slot, int64_t sl, uint2* stk,
+                                           TravCount& tc) {
     jobs.run_lane(true, jobs.job_of(P.job, slot), [&](const DevScene& S, const RParams&) {
         float4 o4 = P.sh_o[sl], d4 = P.sh_d[sl];
         f3 org = f3of(o4), dir = f3of(d4);
@@ -2254,6 +2416,48 @@ __global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_shadow(JOBS jobs, PathBu
         f3 c = f3of(P.sh_c[sl]) * thr;
         P.sh_r[sl] = make_float4(c.x, c.y, c.z, 0.0f);
     });
+}
+
+// The thread's record of the shadow queue; false past its end.  Block b
+// works on the stripes that its XCD (b mod 8) filled, 64 entries of one
+// segment at a time.
+inline unsigned shadow_grid(const PathBufs& P, int maxs) {
+    const int chunks = (P.n + P.chunk - 1) / P.chunk;
+    return (unsigned)(kStripes * ((int64_t)((chunks + kStripes - 1) / kStripes) * P.chunk / kBlock * maxs + maxs));
+}
+__device__ __forceinline__ bool shadow_entry(const PathBufs& P, int maxs, int64_t& sl) {
+    const int lane = (int)threadIdx.x;
+    const int stripes = shadow_stripes(maxs), nseg = (maxs <= kMaxSeg ? maxs : 1) * stripes;
+    // blocks of the lane's segment that are this block's stripe's (with fewer
+    // than 8 stripes the blocks of a stripe take turns)
+    const int x = (int)(blockIdx.x % (unsigned)stripes), turn = (int)(blockIdx.x / (unsigned)stripes);
+    const int count = lane < nseg && lane % stripes == x ? P.seg[lane * kSegStride] : 0;
+    int blocks = (count + kBlock - 1) / kBlock, incl = blocks;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += y;
+    }
+    const unsigned long long past = __ballot(incl > turn);
+    if (past == 0ull) return false;
+    const int s = __ffsll((long long)past) - 1;
+    const int i = (turn - (__shfl(incl, s, 64) - __shfl(blocks, s, 64))) * kBlock + lane;
+    if (i >= __shfl(count, s, 64)) return false;
+    sl = P.q_sh[(int64_t)P.q_seg * s + i];
+    return true;
+}
+
+template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
+__global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_shadow(JOBS jobs, PathBufs P, int maxs) {
+    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
+    uint2 priv_stk[PRIV ? SD : 1];
+    uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
+    constexpr int STRIDE = PRIV ? 1 : kBlock;
+    TravCount tc{0u, 0u, 0u};
+    int64_t sl;
+    if (shadow_entry(P, maxs, sl)) {
+        const int slot = (int)(sl % P.n);
+        shadow_ray<JOBS, SD, STRIDE, COUNT, XF>(jobs, P, slot, sl, stk, tc);
+    }
     if (COUNT) flush_counts(P.tcount + 3, tc);
 }
 
@@ -2262,24 +2466,8 @@ __global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_shadow(JOBS jobs, PathBu
 // record's result is its full contribution or zero).  Same queue view as
 // k_shadow.
 __global__ void __launch_bounds__(kBlock) k_adj_nee(PathBufs P, int maxs, int tex_w, int tex_h) {
-    const bool grouped = maxs <= kMaxSeg;
-    int total = grouped ? 0 : P.counters[kCntShadow];
-    if (grouped)
-        for (int j = 0; j < maxs; j++) total += P.counters[kCntSeg + j];
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= total) return;
-    int64_t qi = i;
-    if (grouped) {
-        int j = 0, pre = 0;
-        for (;;) {
-            int c = P.counters[kCntSeg + j];
-            if (i < pre + c || j + 1 >= maxs) break;
-            pre += c;
-            j++;
-        }
-        qi = (int64_t)j * P.n + (i - pre);
-    }
-    const int64_t sl = P.q_sh[qi];
+    int64_t sl;
+    if (!shadow_entry(P, maxs, sl)) return;
     const float4 g1 = P.adj_g[2 * sl + 1];
     if (g1.w == 0.0f) return;
     const float4 r = P.sh_r[sl];
@@ -2292,7 +2480,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_nee(PathBufs P, int maxs, int te
 // Ends the path in slot p: folds its last shadow results and stores the
 // camera sample's radiance L = w0 * (Le0 + Ld0 + clampInd(Lind)), clamped
 // (Renderer.cs:658-666, 1222-1223), and its AOV probe, under its sample id.
-__device__ __forceinline__ void finish_path(const RParams& R, PathBufs& P, int p) {
+__device__ __forceinline__ void finish_path(const RParams& R, const PathBufs& P, int p) {
     int32_t flags = __float_as_int(P.d[p].w);
     fold_shadows(P, R, p, flags);
     f3 a0 = f3of(P.a0[p]), ai = f3of(P.ai[p]), w0 = f3of(P.w0[p]);
@@ -2332,61 +2520,107 @@ __device__ __forceinline__ void finish_path(const RParams& R, PathBufs& P, int p
 // sample does not change any result.
 template <class JOBS>
 __global__ void __launch_bounds__(kBlock) k_retire(JOBS jobs, PathBufs P) {
-    const int p = xcd_block() * kBlock + threadIdx.x;
-    const bool ret = p < P.n && P.state[p] == kSlotRetired;
-    if (ret) finish_path(jobs.params(jobs.job_of(P.job, p)), P, p);
+    __shared__ ChunkLds<1, kChunkOne> lds;
+    const int base = chunk_base(P.chunk);
+    const ChunkList L = chunk_list(P.state, base, P.n, P.chunk, lds,
+                                   [](uint8_t st) { return st == kSlotRetired ? 0 : -1; });
     const int ws = P.counters[kCntWs];
-    const unsigned long long lt = (1ull << (threadIdx.x & 63)) - 1ull;
-    const unsigned long long rb = __ballot(ret);
-    const int sid = P.counters[kCntSidBase] + P.wc[kWcRetire * P.nw + (p >> 6)] + __popcll(rb & lt);
-    bool start = ret && sid < ws;
-    if (ret) {
-        int st = kSlotIdle;
-        if (start) {
+    const int sid0 = P.counters[kCntSidBase] + P.wc[kWcRetire * P.nw + base / P.chunk];
+    for (int t = threadIdx.x; t < L.n0; t += kBlock) {
+        const int p = base + L.q[t], sid = sid0 + t;
+        finish_path(jobs.params(jobs.job_of(P.job, p)), P, p);
+        uint8_t st = kSlotIdle;
+        if (sid < ws) {
             int job, pix, pass;
             resolve_sample(P, sid, job, pix, pass);
             const RParams& R = jobs.params(job);
             init_path(jobs.scene(job), R, P, p, sid, job, pix, pass);
-            st = R.max_depth > 0 ? kSlotActive : kSlotRetired;
+            st = R.max_depth > 0 ? kSlotFresh : kSlotRetired;
         }
         P.state[p] = st;
+        P.smask[p] = 0;     // an idle slot queues no shadow rays
+        if (P.q_g) P.gflag[p] = 0;
     }
 }
 
 // Per-pixel film accumulation in sample order (Renderer.cs:668-672,
 // CaptureAccumulator.Add, Renderer.cs:829-856): the window's samples of a
 // pixel are summed pass by pass, even passes into half A, odd into half B.
+// A wave sums 64 pixels (a run of the window's pixel order), kAccRun samples
+// of each at a time: they are fetched as whole 128-byte lines and turned
+// through LDS, so each lane then adds its own pixel's in order.
+constexpr int kAccRun = 8;
+struct AccTile {
+    float4 v[kBlock][kAccRun + 1];
+    // samples [s0, s0 + n) of pixels [q0, q0 + kBlock) of `src`
+    __device__ __forceinline__ void load(const float4* __restrict__ src, int64_t q0, int npix, int passes, int s0, int n) {
+#pragma unroll
+        for (int k = 0; k < kAccRun; k++) {
+            const int i = k * kBlock + (int)threadIdx.x, px = i / kAccRun, s = i % kAccRun;
+            if (s < n && q0 + px < npix) v[px][s] = src[(q0 + px) * passes + s0 + s];
+        }
+    }
+};
+template <bool AOVS>
 __global__ void __launch_bounds__(kBlock) k_accum(RParams R, PathBufs P, FilmBufs F, int pass0, int passes, int off) {
-    const int q = blockIdx.x * kBlock + threadIdx.x;
-    if (q >= R.npix) return;
-    const int np = R.npix, pix = pixel_of_rank(q, R.W, np);
-    f3 sum = mk(F.sum[pix], F.sum[np + pix], F.sum[2 * np + pix]);
-    f3 sa = mk(F.sa[pix], F.sa[np + pix], F.sa[2 * np + pix]);
-    f3 sb = mk(F.sb[pix], F.sb[np + pix], F.sb[2 * np + pix]);
-    for (int sl = 0; sl < passes; sl++) {
-        int s = R.soff + pass0 + sl;
-        int64_t k = (int64_t)off + (int64_t)q * passes + sl;
-        float4 l = P.res_l[k];
-        f3 L = f3of(l);
-        sum += L;
-        bool isA = (s & 1) == 0;
-        if (isA) sa += L;
-        else sb += L;
-        if (R.aovs) {
-            f3 alb = f3of(P.res_a[k]), nrm = f3of(P.res_n[k]);
-            float* A = isA ? F.alba : F.albb;
-            float* N = isA ? F.nrma : F.nrmb;
-            A[pix] += alb.x; A[np + pix] += alb.y; A[2 * np + pix] += alb.z;
-            N[pix] += nrm.x; N[np + pix] += nrm.y; N[2 * np + pix] += nrm.z;
-            if (l.w >= 0.0f) {
-                if (isA) { F.depa[pix] += l.w; F.dca[pix]++; }
-                else { F.depb[pix] += l.w; F.dcb[pix]++; }
+    __shared__ AccTile tl, aov[AOVS ? 2 : 1];   // radiance; albedo, normal
+    const int64_t q0 = (int64_t)blockIdx.x * kBlock;
+    const int q = (int)q0 + (int)threadIdx.x, np = R.npix;
+    const bool on = q < np;
+    const int pix = on ? pixel_of_rank(q, R.W, np) : 0;
+    auto get3 = [&](const float* p) { return mk(p[pix], p[np + pix], p[2 * np + pix]); };
+    auto put3 = [&](float* p, f3 v) { p[pix] = v.x; p[np + pix] = v.y; p[2 * np + pix] = v.z; };
+    f3 sum = get3(F.sum), sa = get3(F.sa), sb = get3(F.sb);
+    f3 alba = splat(0.0f), albb = alba, nrma = alba, nrmb = alba;
+    float depa = 0.0f, depb = 0.0f;
+    int dca = 0, dcb = 0;
+    if (AOVS) {
+        alba = get3(F.alba), albb = get3(F.albb), nrma = get3(F.nrma), nrmb = get3(F.nrmb);
+        depa = F.depa[pix], depb = F.depb[pix], dca = F.dca[pix], dcb = F.dcb[pix];
+    }
+    for (int s0 = 0; s0 < passes; s0 += kAccRun) {
+        const int n = min(kAccRun, passes - s0);
+        __syncthreads();
+        tl.load(P.res_l + off, q0, np, passes, s0, n);
+        if (AOVS) {
+            aov[0].load(P.res_a + off, q0, np, passes, s0, n);
+            aov[1].load(P.res_n + off, q0, np, passes, s0, n);
+        }
+        __syncthreads();
+        for (int k = 0; k < n; k++) {
+            const float4 l = tl.v[threadIdx.x][k];
+            const f3 L = f3of(l);
+            sum += L;
+            const bool isA = ((R.soff + pass0 + s0 + k) & 1) == 0;
+            if (isA) sa += L;
+            else sb += L;
+            if (AOVS) {
+                const f3 alb = f3of(aov[0].v[threadIdx.x][k]), nrm = f3of(aov[1].v[threadIdx.x][k]);
+                if (isA) {
+                    alba += alb;
+                    nrma += nrm;
+                } else {
+                    albb += alb;
+                    nrmb += nrm;
+                }
+                if (l.w >= 0.0f) {
+                    if (isA) { depa += l.w; dca++; }
+                    else { depb += l.w; dcb++; }
+                }
             }
         }
     }
-    F.sum[pix] = sum.x; F.sum[np + pix] = sum.y; F.sum[2 * np + pix] = sum.z;
-    F.sa[pix] = sa.x; F.sa[np + pix] = sa.y; F.sa[2 * np + pix] = sa.z;
-    F.sb[pix] = sb.x; F.sb[np + pix] = sb.y; F.sb[2 * np + pix] = sb.z;
+    if (!on) return;
+    put3(F.sum, sum);
+    put3(F.sa, sa);
+    put3(F.sb, sb);
+    if (AOVS) {
+        put3(F.alba, alba);
+        put3(F.albb, albb);
+        put3(F.nrma, nrma);
+        put3(F.nrmb, nrmb);
+        F.depa[pix] = depa, F.depb[pix] = depb, F.dca[pix] = dca, F.dcb[pix] = dcb;
+    }
 }
 
 __global__ void k_resolve(RParams R, FilmBufs F, float exposure) {
@@ -2692,38 +2926,38 @@ static DevScene dev_view(const rt_scene* sc) {
 // Launches a traversal kernel with the LDS stack depth the scene needs.
 // Traversal kernels: job source J, stack depth, traversal counting, stack
 // placement (batches always use the private stack).
-#define DISPATCH_SD_C(J, sd, cnt, priv, KERNEL, grid, ...)                                            \
+#define DISPATCH_SD_C(J, sd, cnt, priv, KERNEL, grid, bs, ...)                                            \
     do {                                                                                               \
         if constexpr (std::is_same<J, OneJob>::value) {                                                \
             if (cnt) {                                                                                 \
-                if (priv) DISPATCH_SD_T(J, sd, KERNEL, true, true, grid, __VA_ARGS__);                 \
-                else DISPATCH_SD_T(J, sd, KERNEL, true, false, grid, __VA_ARGS__);                     \
+                if (priv) DISPATCH_SD_T(J, sd, KERNEL, true, true, grid, bs, __VA_ARGS__);                 \
+                else DISPATCH_SD_T(J, sd, KERNEL, true, false, grid, bs, __VA_ARGS__);                     \
             } else {                                                                                   \
-                if (priv) DISPATCH_SD_T(J, sd, KERNEL, false, true, grid, __VA_ARGS__);                \
-                else DISPATCH_SD_T(J, sd, KERNEL, false, false, grid, __VA_ARGS__);                    \
+                if (priv) DISPATCH_SD_T(J, sd, KERNEL, false, true, grid, bs, __VA_ARGS__);                \
+                else DISPATCH_SD_T(J, sd, KERNEL, false, false, grid, bs, __VA_ARGS__);                    \
             }                                                                                          \
         } else {                                                                                       \
-            if (cnt) DISPATCH_SD_T(J, sd, KERNEL, true, true, grid, __VA_ARGS__);                      \
-            else DISPATCH_SD_T(J, sd, KERNEL, false, true, grid, __VA_ARGS__);                         \
+            if (cnt) DISPATCH_SD_T(J, sd, KERNEL, true, true, grid, bs, __VA_ARGS__);                      \
+            else DISPATCH_SD_T(J, sd, KERNEL, false, true, grid, bs, __VA_ARGS__);                         \
         }                                                                                              \
     } while (0)
-#define DISPATCH_SD_T(J, sd, KERNEL, C_, P_, grid, ...)                                                        \
+#define DISPATCH_SD_T(J, sd, KERNEL, C_, P_, grid, bs, ...)                                                 \
     do {                                                                                                       \
-        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<J, 24, C_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);       \
-        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<J, 32, C_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);  \
-        else hipLaunchKernelGGL((KERNEL<J, 64, C_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);                  \
+        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<J, 24, C_, P_>), grid, dim3(bs), 0, __VA_ARGS__);       \
+        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<J, 32, C_, P_>), grid, dim3(bs), 0, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((KERNEL<J, 64, C_, P_>), grid, dim3(bs), 0, __VA_ARGS__);                  \
     } while (0)
 // scenes with wrapper entries: the XF traversal, private-scratch stacks
-#define DISPATCH_SD_X(J, sd, cnt, KERNEL, grid, ...)                                   \
+#define DISPATCH_SD_X(J, sd, cnt, KERNEL, grid, bs, ...)                                   \
     do {                                                                                \
-        if (cnt) DISPATCH_SD_TX(J, sd, KERNEL, true, grid, __VA_ARGS__);                \
-        else DISPATCH_SD_TX(J, sd, KERNEL, false, grid, __VA_ARGS__);                   \
+        if (cnt) DISPATCH_SD_TX(J, sd, KERNEL, true, grid, bs, __VA_ARGS__);                \
+        else DISPATCH_SD_TX(J, sd, KERNEL, false, grid, bs, __VA_ARGS__);                   \
     } while (0)
-#define DISPATCH_SD_TX(J, sd, KERNEL, C_, grid, ...)                                                                 \
+#define DISPATCH_SD_TX(J, sd, KERNEL, C_, grid, bs, ...)                                                          \
     do {                                                                                                             \
-        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<J, 24, C_, true, true>), grid, dim3(kBlock), 0, __VA_ARGS__);      \
-        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<J, 32, C_, true, true>), grid, dim3(kBlock), 0, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERNEL<J, 64, C_, true, true>), grid, dim3(kBlock), 0, __VA_ARGS__);                 \
+        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<J, 24, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__);      \
+        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<J, 32, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__); \
+        else hipLaunchKernelGGL((KERNEL<J, 64, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__);                 \
     } while (0)
 #define DISPATCH_SD(sd, KERNEL, grid, ...)                                                       \
     do {                                                                                         \
@@ -2773,7 +3007,8 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
         all_lights = jobs.all_lights != 0;
     }
     const int pool_blocks = (int)((N + kBlock - 1) / kBlock);
-    const int shadow_blocks = (int)(((int64_t)N * maxs + kBlock - 1) / kBlock);
+    const int chunks = (int)((N + P.chunk - 1) / P.chunk);
+    const unsigned shadow_blocks = shadow_grid(P, maxs);
     size_t pbytes = sizeof(PartDev) * std::max<size_t>(plan.parts.size(), 1);
     if (pbytes > ctx->parts_bytes) {
         if (ctx->parts_mem) hipFree(ctx->parts_mem);
@@ -2786,14 +3021,13 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(hipMemcpy(d_parts, plan.parts.data(), sizeof(PartDev) * plan.parts.size(), hipMemcpyHostToDevice));
     auto enqueue_iteration = [&](const PathBufs& Pw, hipEvent_t* e) -> int {
-        hipLaunchKernelGGL(k_iter_begin, dim3(1), dim3(kBlock), 0, ctx->stream, Pw, traced ? 1 : 0);
         if (traced) {
-            dim3 grid(pool_blocks);
+            const dim3 grid(chunks);
             if (e) HIP_TRY(hipEventRecord(e[0], ctx->stream));
-            if (hier) DISPATCH_SD_X(JOBS, stack_depth, counting, k_trace, grid, ctx->stream, jobs, Pw);
-            else DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_trace, grid, ctx->stream, jobs, Pw);
+            if (hier) DISPATCH_SD_X(JOBS, stack_depth, counting, k_trace, dim3((unsigned)((N + P.wide - 1) / P.wide)), kWg, ctx->stream, jobs, Pw);
+            else DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_trace, dim3((unsigned)((N + P.wide - 1) / P.wide)), kWg, ctx->stream, jobs, Pw);
             if (e) HIP_TRY(hipEventRecord(e[1], ctx->stream));
-            if (Pw.fp) DISPATCH_SD_C(JOBS, stack_depth, false, ctx->priv_stack, k_fp, grid, ctx->stream, jobs, Pw);
+            if (Pw.fp) DISPATCH_SD_C(JOBS, stack_depth, false, ctx->priv_stack, k_fp, dim3(pool_blocks), kBlock, ctx->stream, jobs, Pw);
             bool adj_replay = false;
             if constexpr (std::is_same<JOBS, OneJob>::value) adj_replay = Pw.adj_pass == 2;
             if (adj_replay) {
@@ -2819,21 +3053,26 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                                                0, ctx->stream, jobs, Pw, maxs);
                     }
                 } else {
+                    const bool wide = N >= kNeeWide;
+                    const dim3 ngrid(wide ? (unsigned)((N + P.wide - 1) / P.wide) : (unsigned)chunks);
+                    const dim3 nblk(wide ? kWg : kBlock);
+#define LAUNCH_NEE(W_, UL_)                                                                                          \
+    do {                                                                                                             \
+        if (wide)                                                                                                    \
+            hipLaunchKernelGGL((k_shade<JOBS, W_, false, kPhNee, true, false, UL_, kWaves>), ngrid, nblk, 0,         \
+                               ctx->stream, jobs, Pw, maxs);                                                         \
+        else                                                                                                         \
+            hipLaunchKernelGGL((k_shade<JOBS, W_, false, kPhNee, true, false, UL_, 1>), ngrid, nblk, 0, ctx->stream, \
+                               jobs, Pw, maxs);                                                                      \
+    } while (0)
                     if (ctx->shade_wpe <= 2) {
-                        if (all_lights)
-                            hipLaunchKernelGGL((k_shade<JOBS, 2, false, kPhNee, true, false, true>), grid, dim3(kBlock),
-                                               0, ctx->stream, jobs, Pw, maxs);
-                        else
-                            hipLaunchKernelGGL((k_shade<JOBS, 2, false, kPhNee>), grid, dim3(kBlock), 0, ctx->stream,
-                                               jobs, Pw, maxs);
+                        if (all_lights) LAUNCH_NEE(2, true);
+                        else LAUNCH_NEE(2, false);
                     } else {
-                        if (all_lights)
-                            hipLaunchKernelGGL((k_shade<JOBS, 3, false, kPhNee, true, false, true>), grid, dim3(kBlock),
-                                               0, ctx->stream, jobs, Pw, maxs);
-                        else
-                            hipLaunchKernelGGL((k_shade<JOBS, 3, false, kPhNee>), grid, dim3(kBlock), 0, ctx->stream,
-                                               jobs, Pw, maxs);
+                        if (all_lights) LAUNCH_NEE(3, true);
+                        else LAUNCH_NEE(3, false);
                     }
+#undef LAUNCH_NEE
                     if (thin_film) {
                         if (ctx->bounce_wpe <= 2)
                             hipLaunchKernelGGL((k_shade<JOBS, 2, false, kPhBounce, true>), grid, dim3(kBlock), 0,
@@ -2852,14 +3091,12 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                 }
             }
             if (e) HIP_TRY(hipEventRecord(e[2], ctx->stream));
-            hipLaunchKernelGGL(k_wave_scan, dim3(kWcSeg + (maxs <= kMaxSeg ? maxs : 0)), dim3(1024), 0, ctx->stream, Pw);
-            hipLaunchKernelGGL(k_compact, grid, dim3(kBlock), 0, ctx->stream, Pw, maxs);
-            if (gather_scene) hipLaunchKernelGGL(k_gather, grid, dim3(kBlock), 0, ctx->stream, *gather_scene, Pw, *M);
+            if (gather_scene) hipLaunchKernelGGL(k_gather, dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, *gather_scene, Pw, *M);
             if (e) HIP_TRY(hipEventRecord(e[3], ctx->stream));
             if (hier)
-                DISPATCH_SD_X(JOBS, stack_depth, counting, k_shadow, dim3(shadow_blocks), ctx->stream, jobs, Pw, maxs);
+                DISPATCH_SD_X(JOBS, stack_depth, counting, k_shadow, dim3(shadow_blocks), kBlock, ctx->stream, jobs, Pw, maxs);
             else
-                DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_shadow, dim3(shadow_blocks), ctx->stream,
+                DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_shadow, dim3(shadow_blocks), kBlock, ctx->stream,
                               jobs, Pw, maxs);
             if (e) HIP_TRY(hipEventRecord(e[4], ctx->stream));
             if constexpr (std::is_same<JOBS, OneJob>::value)
@@ -2867,11 +3104,10 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                     hipLaunchKernelGGL(k_adj_nee, dim3(shadow_blocks), dim3(kBlock), 0, ctx->stream, Pw, maxs, jobs.S.tex_w,
                                        jobs.S.tex_h);
         } else {
-            const int narr = kWcSeg + (maxs <= kMaxSeg ? maxs : 0);
-            hipLaunchKernelGGL(k_count_retired, dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, Pw, narr);
-            hipLaunchKernelGGL(k_wave_scan, dim3(narr), dim3(1024), 0, ctx->stream, Pw);
+            hipLaunchKernelGGL(k_count_retired, dim3(chunks), dim3(kBlock), 0, ctx->stream, Pw);
         }
-        hipLaunchKernelGGL((k_retire<JOBS>), dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw);
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, ctx->stream, Pw, traced ? 1 : 0);
+        hipLaunchKernelGGL((k_retire<JOBS>), dim3(chunks), dim3(kBlock), 0, ctx->stream, jobs, Pw);
         HIP_TRY(hipGetLastError());
         return RT_OK;
     };
@@ -2895,9 +3131,10 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
         const int ws = plan.ws[w];
         const int n0 = (int)std::min<int64_t>(N, ws);
         HIP_TRY(hipMemsetAsync(P.counters, 0, 4 * kCntWindow, ctx->stream));
-        hipLaunchKernelGGL((k_raygen<JOBS>), dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw, n0, ws);
+        hipLaunchKernelGGL((k_raygen<JOBS>), dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw, n0, ws,
+                           traced ? 1 : 0);
         // graph mode: the kIterBatch iterations of a batch are captured once
-        // per window (no memset nodes: k_iter_begin clears the counters) and
+        // per window (no memset nodes: k_scan and k_raygen clear the counters) and
         // replayed; per-kernel timings are not recorded
         hipGraphExec_t gexec = nullptr;
         if (ctx->use_graph) {
@@ -2937,7 +3174,6 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                 }
                 nb[set] = gexec ? 0 : iters;
             }
-            hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(kBlock), 0, ctx->stream, Pw);
             HIP_TRY(hipMemcpyAsync(&ctx->pinned[4 * set], &P.counters[kCntPend], 12, hipMemcpyDeviceToHost,
                                    ctx->stream));
             HIP_TRY(hipEventRecord(ctx->chk[set], ctx->stream));
@@ -3632,11 +3868,19 @@ int rt_photon_gather(rt_ctx* ctx, const rt_scene* sc, const rt_settings* s, cons
 // in the context's grow-only buffer.
 static int alloc_paths(rt_ctx* ctx, int64_t N, int64_t WS, int maxs, bool aovs, bool gather, bool fp, bool xf,
                        PathBufs& P) {
-    size_t per_path = 8 * 16 + 8 * 4 + 4 + 16 + (aovs ? 5 * 16 : 0) + 4 * 16 * (size_t)maxs + 8 * 4 + 4 * (size_t)maxs +
-                      (gather ? 64 : 0) + (fp ? 16 : 0) + (xf ? 16 : 0);
+    const int chunk = chunk_one(N);
+    const size_t nch = (size_t)(((N + chunk - 1) / chunk + 3) & ~(int64_t)3);   // row stride of the counts (int4 rows)
+    size_t per_path = 8 * 16 + 8 * 4 + 4 + 16 + (aovs ? 5 * 16 : 0) + 4 * 16 * (size_t)maxs + 1 + 5 * 4 +
+                      (gather ? 69 : 0) + (fp ? 16 : 0) + (xf ? 16 : 0);
+    // a stripe of a segment holds every chunk of its workgroups (times the
+    // light samples in the ungrouped form)
+    const int stripes = shadow_stripes(maxs);
+    const int64_t stripe_slots = (((N + chunk - 1) / chunk + stripes - 1) / stripes) * chunk;
+    const int64_t q_seg = stripe_slots * (maxs <= kMaxSeg ? 1 : maxs);
+    const size_t q_all = (size_t)q_seg * stripes * (maxs <= kMaxSeg ? maxs : 1);
     size_t per_sample = aovs ? 48 : 16;
-    size_t need = (size_t)N * per_path + (size_t)WS * per_sample + 40 * 256 + 16384 + 8 * N +
-                  4 * (size_t)((N + kBlock - 1) / kBlock + 3) * (kWcSeg + kMaxSeg);
+    size_t need = (size_t)N * per_path + (size_t)WS * per_sample + 40 * 256 + 16384 +
+                  4 * kWcRows * nch + 4 * kSegStride * kSegs + 4 * q_all;
     if (need > ctx->path_bytes) {
         if (ctx->path_mem) hipFree(ctx->path_mem);
         ctx->path_mem = nullptr;
@@ -3677,19 +3921,23 @@ static int alloc_paths(rt_ctx* ctx, int64_t N, int64_t WS, int maxs, bool aovs, 
     P.sh_d = (float4*)take(16 * N * maxs);
     P.sh_c = (float4*)take(16 * N * maxs);
     P.sh_r = (float4*)take(16 * N * maxs);
-    P.q_sh = (int32_t*)take(4 * N * maxs);
-    P.state = (int32_t*)take(4 * N);
+    P.state = (uint8_t*)take(N);
     P.smask = (int32_t*)take(4 * N);
-    P.gflag = (int32_t*)take(4 * N);
-    P.q_g = (int32_t*)take(4 * N);
-    P.nw = (int)(((N + kBlock - 1) / kBlock + 3) & ~(int64_t)3);   // row stride of the count arrays (int4 rows)
-    P.wc = (int32_t*)take(4 * (size_t)P.nw * (kWcSeg + std::min(maxs, kMaxSeg)));
+    P.wide = chunk_wide(N);
+    P.chunk = chunk;
+    P.nw = (int)nch;
+    P.wc = (int32_t*)take(4 * kWcRows * nch);
+    P.q_seg = (int)q_seg;
+    P.q_sh = (int32_t*)take(4 * q_all);
+    P.seg = (int32_t*)take(4 * kSegStride * kSegs);
     P.job = (int32_t*)take(4 * N);
     P.pix = (int32_t*)take(4 * N);
     P.pass = (int32_t*)take(4 * N);
     P.sid = (int32_t*)take(4 * N);
     P.res_l = (float4*)take(16 * WS);
     if (gather) {
+        P.gflag = (uint8_t*)take(N);
+        P.q_g = (int32_t*)take(4 * N);
         P.gq0 = (float4*)take(16 * N);
         P.gq1 = (float4*)take(16 * N);
         P.gq2 = (float4*)take(16 * N);
@@ -3737,6 +3985,14 @@ static size_t film_layout(char* base, int64_t npix, FilmBufs& F, size_t* acc_byt
     F.out_depa = (float*)ftake(4 * (size_t)npix);
     F.out_depb = (float*)ftake(4 * (size_t)npix);
     return off;
+}
+
+static void launch_accum(rt_ctx* ctx, const RParams& R, const PathBufs& P, const FilmBufs& F, const PartDev& pt) {
+    const dim3 grid((unsigned)((pt.npix + kBlock - 1) / kBlock));
+    if (R.aovs)
+        hipLaunchKernelGGL(k_accum<true>, grid, dim3(kBlock), 0, ctx->stream, R, P, F, pt.pass0, pt.npass, pt.off);
+    else
+        hipLaunchKernelGGL(k_accum<false>, grid, dim3(kBlock), 0, ctx->stream, R, P, F, pt.pass0, pt.npass, pt.off);
 }
 
 static int grow(rt_ctx* ctx, void** mem, size_t* bytes, size_t need) {
@@ -3939,10 +4195,7 @@ int rt_render(rt_ctx* ctx, const rt_scene* sc, const rt_settings* s, const rt_fi
     OneJob one{S, R};
     rc = run_windows(ctx, one, P, maxs, s->max_depth > 0, counting, sc->stack_depth, S.caustics ? &S : nullptr, &PP.M,
                      plan,
-                     [&](const PartDev& pt) {
-                         hipLaunchKernelGGL(k_accum, dim3((npix + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream,
-                                            R, P, F, pt.pass0, pt.npass, pt.off);
-                     },
+                     [&](const PartDev& pt) { launch_accum(ctx, R, P, F, pt); },
                      tm);
     if (rc) return rc;
     const double t_trace = tm.trace, t_shade = tm.shade, t_shadow = tm.shadow;
@@ -4211,11 +4464,7 @@ int rt_render_batch(rt_ctx* ctx, const rt_batch_job* jobs, int32_t n_jobs, int32
         many.hier |= jd[j].S.xf != nullptr ? 1 : 0;
         if (R[j].picked) many.all_lights = 0;
     }
-    auto accum = [&](const PartDev& pt) {
-        const int64_t npix = pt.npix;
-        hipLaunchKernelGGL(k_accum, dim3((unsigned)((npix + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
-                           R[pt.job], P, F[pt.job], pt.pass0, pt.npass, pt.off);
-    };
+    auto accum = [&](const PartDev& pt) { launch_accum(ctx, R[pt.job], P, F[pt.job], pt); };
     for (const Segment& sg : segs) {
         if (sg.job >= 0) {
             OneJob one{jd[sg.job].S, R[sg.job]};

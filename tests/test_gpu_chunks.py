@@ -1,0 +1,88 @@
+"""Pool chunking: a film does not depend on the pool size, so every chunk
+shape (one slot, less and more than a wave, several rows, the four-wave NEE
+phase of large pools) must give the same bits; shadow-queue forms (one to
+eight, sixteen and thirty-two light samples a vertex take different stripe
+counts, more take the ungrouped queue) and odd image sizes (partial 8-row
+strips) follow the oracle."""
+import numpy as np
+import pytest
+
+from raytracer import abi, native, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(W, H, samples):
+    """A corner lit by area lights with `samples` shadow samples in all
+    (squares of 1 and 4 a light).  Area lights are sampled without
+    trigonometry: a sphere light's limb samples flip with the last bit of
+    cosf, which differs between the device and the C library."""
+    b = scenes.SceneBuilder()
+    white = b.lambertian((0.7, 0.7, 0.7))
+    shiny = b.disney((0.6, 0.3, 0.2), roughness=0.3)
+    b.quad((-3, 0, -3), (0, 0, 6), (6, 0, 0), white)
+    b.quad((-3, 0, -3), (6, 0, 0), (0, 6, 0), white)
+    b.sphere((-0.6, 0.6, 0.0), 0.6, shiny)
+    b.sphere((0.7, 0.4, 0.5), 0.4, white)
+    left, k = samples, 0
+    while left > 0:
+        ss = 4 if left >= 4 else 1
+        ang = 0.7 * k
+        b.area_light((2.0 * np.cos(ang), 3.0 + 0.1 * k, 2.0 * np.sin(ang)), (0.3, 0.0, 0.0), (0.0, 0.0, 0.3),
+                     intensity=12.0, shadow_samples=ss)
+        left, k = left - ss, k + 1
+    return b.build(scenes.make_camera((0.0, 1.5, 5.0), (0.0, 0.7, 0.0), 45.0, W / H))
+
+
+def _film(sc, W, H, spp, pool, aovs=True):
+    return native.Renderer(sc, spp, 4, paths_in_flight=pool).render(W, H, capture_aovs=aovs).buffers
+
+
+PLANES = ("beauty", "beauty_a", "beauty_b", "albedo_a", "albedo_b", "normal_a", "normal_b", "depth_a", "depth_b")
+
+
+@pytest.mark.parametrize("samples", [1, 8, 9, 17, 32, 40])
+def test_pool_sizes_and_queue_forms(gpu_ctx, oracle, samples):
+    W, H, spp = 37, 19, 3
+    desc = _scene(W, H, samples)
+    sc = native.Scene(gpu_ctx, desc)
+    try:
+        ref = _film(sc, W, H, spp, 0)
+        for pool in (1 if samples == 1 else 61, 64, 65, 257, 1000):
+            got = _film(sc, W, H, spp, pool)
+            for k in PLANES:
+                assert np.array_equal(getattr(ref, k), getattr(got, k)), (samples, pool, k)
+        st = abi.settings_defaults(W, H, spp, 4)
+        o = oracle.OracleScene(desc).render(st)["beauty"]
+    finally:
+        sc.close()
+    err = np.abs(ref.beauty - o) / np.maximum(np.abs(o), 1e-2)
+    print(f"{samples} samples a vertex: {np.mean(err < 1e-3):.4f} of the values within 1e-3, max {err.max():.2e}", flush=True)
+    assert np.mean(err < 1e-3) > 0.99
+
+
+@pytest.mark.parametrize("size", [(1, 1), (3, 200), (200, 3), (65, 8), (64, 9)])
+def test_image_shapes(gpu_ctx, oracle, size):
+    W, H = size
+    desc = _scene(W, H, 2)
+    sc = native.Scene(gpu_ctx, desc)
+    try:
+        ref = _film(sc, W, H, 5, 0)
+    finally:
+        sc.close()
+    o = oracle.OracleScene(desc).render(abi.settings_defaults(W, H, 5, 4))["beauty"]
+    err = np.abs(ref.beauty - o) / np.maximum(np.abs(o), 1e-2)
+    assert np.mean(err < 1e-3) > 0.99, (size, err.max())
+
+
+def test_wide_nee_pool(gpu_ctx):
+    # 5.2 M samples: the default pool runs the NEE phase four waves wide
+    W = H = 1024
+    sc = native.Scene(gpu_ctx, _scene(W, H, 2))
+    try:
+        a = _film(sc, W, H, 5, 0, aovs=False)
+        b = _film(sc, W, H, 5, 1 << 20, aovs=False)
+    finally:
+        sc.close()
+    for k in ("beauty", "beauty_a", "beauty_b"):
+        assert np.array_equal(getattr(a, k), getattr(b, k)), k
