@@ -291,16 +291,18 @@ __global__ void __launch_bounds__(kBlock) k_photon_compact(int ntot, const int32
     ow[k] = iw[g];
 }
 
-// Component-wise min of the photon positions (exact in any order):
+// Component-wise min or max of the photon positions (exact in any order):
 // per-block partials, then one block folds the partials.
-__global__ void __launch_bounds__(256) k_min3(const float4* __restrict__ p, int n, float4* __restrict__ part) {
+template <bool MAX>
+__global__ void __launch_bounds__(256) k_bound3(const float4* __restrict__ p, int n, float4* __restrict__ part) {
     __shared__ float sm[3][256];
-    float mx = __int_as_float(0x7f800000), my = mx, mz = mx;
+    auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : fminf(a, b); };
+    float mx = __int_as_float(MAX ? 0xff800000 : 0x7f800000), my = mx, mz = mx;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         float4 q = p[i];
-        mx = fminf(mx, q.x);
-        my = fminf(my, q.y);
-        mz = fminf(mz, q.z);
+        mx = op(mx, q.x);
+        my = op(my, q.y);
+        mz = op(mz, q.z);
     }
     sm[0][threadIdx.x] = mx;
     sm[1][threadIdx.x] = my;
@@ -308,7 +310,7 @@ __global__ void __launch_bounds__(256) k_min3(const float4* __restrict__ p, int 
     __syncthreads();
     for (int s = 128; s > 0; s >>= 1) {
         if (threadIdx.x < s)
-            for (int c = 0; c < 3; c++) sm[c][threadIdx.x] = fminf(sm[c][threadIdx.x], sm[c][threadIdx.x + s]);
+            for (int c = 0; c < 3; c++) sm[c][threadIdx.x] = op(sm[c][threadIdx.x], sm[c][threadIdx.x + s]);
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = make_float4(sm[0][0], sm[1][0], sm[2][0], 0.0f);
@@ -413,7 +415,8 @@ struct DevPhotons {
     const float4* spw;      // contiguous run of start[b] .. start[b+1]
     const int32_t* start;
     const int32_t* idx;
-    const float4* origin;   // device scalar (x, y, z)
+    const float4* origin;   // device scalars (x, y, z): smallest position (the grid's origin) and largest
+    const float4* top;
     float cell, inv_cell, max_r;
     uint32_t mask;
     int n;
@@ -481,47 +484,85 @@ __device__ __forceinline__ void heap_insert(float2* h, int& count, int id, float
 // distance is inside the scanned reach.  Returns the count and the kernel
 // radius (distance of the farthest gathered photon); the heap holds
 // bucket-order record indices.
+//
+// Bound by the latency of the cell lookups (a random 8-byte read each, up to
+// 343 a search) at the 2 waves/SIMD the heaps leave.  Cells that cannot hold
+// a photon are not looked up: rows and planes of a shell outside the cells
+// of the photons' bounding box (photons on a floor fill one layer, and a
+// hashed lookup of another layer would fetch other cells' photons), and rows
+// and planes whose distance alone fails the two tests (dx^2 >= 0, and
+// rounding is monotone, so each of their cells would fail them).  The starts
+// of four cells of a row are fetched at once, then their first records.  The visit order of the cells
+// that hold photons, hence the heap, is the reference's.  1280x720 x 32
+// frame with 20 M photons: k_gather 7.78 -> 6.32 ms a launch.
 template <int S>
 __device__ int photon_knn(const DevPhotons& M, f3 p, float2* h, float& radius) {
     radius = 0.0f;
     if (M.n <= 0) return 0;
-    f3 org = f3of(M.origin[0]);
-    int cx, cy, cz;
+    const f3 org = f3of(M.origin[0]);
+    int cx, cy, cz, tx, ty, tz;
     photon_cell(p, org, M.inv_cell, cx, cy, cz);
+    photon_cell(f3of(M.top[0]), org, M.inv_cell, tx, ty, tz);   // cells [0, t] hold every photon
     const float max_r2 = M.max_r * M.max_r;
     int count = 0;
     const int max_rings = (int)ceilf(M.max_r * M.inv_cell) + 1;
+    if (cx < -max_rings || cy < -max_rings || cz < -max_rings || (int64_t)cx > (int64_t)tx + max_rings ||
+        (int64_t)cy > (int64_t)ty + max_rings || (int64_t)cz > (int64_t)tz + max_rings)
+        return 0;
+    auto axis_d = [&](float lo, float q) { return fmaxf(fmaxf(lo - q, q - (lo + M.cell)), 0.0f); };
     for (int ring = 0; ring <= max_rings; ring++) {
-        for (int z = cz - ring; z <= cz + ring; z++)
-            for (int y = cy - ring; y <= cy + ring; y++) {
+        for (int z = max(cz - ring, 0); z <= min(cz + ring, tz); z++) {
+            const float dz = axis_d(org.z + (float)z * M.cell, p.z), dz2 = dz * dz;
+            if (dz2 > max_r2 || (count >= kGatherK && dz2 >= h[0].x)) continue;
+            for (int y = max(cy - ring, 0); y <= min(cy + ring, ty); y++) {
+                const float dy = axis_d(org.y + (float)y * M.cell, p.y), dy2 = dy * dy;
+                if (dy2 + dz2 > max_r2 || (count >= kGatherK && dy2 + dz2 >= h[0].x)) continue;
                 // rows inside the shell hold only its two end cells
                 const bool face = ring == 0 || abs(z - cz) == ring || abs(y - cy) == ring;
                 const int xstep = face ? 1 : 2 * ring;
-                for (int x = cx - ring; x <= cx + ring; x += xstep) {
-                    float bx = org.x + (float)x * M.cell, by = org.y + (float)y * M.cell, bz = org.z + (float)z * M.cell;
-                    float dx = fmaxf(fmaxf(bx - p.x, p.x - (bx + M.cell)), 0.0f);
-                    float dy = fmaxf(fmaxf(by - p.y, p.y - (by + M.cell)), 0.0f);
-                    float dz = fmaxf(fmaxf(bz - p.z, p.z - (bz + M.cell)), 0.0f);
-                    float md2 = (dx * dx + dy * dy) + dz * dz;
-                    if (md2 > max_r2) continue;
-                    if (count >= kGatherK && md2 >= h[0].x) continue;
-                    uint32_t b = photon_bucket(x, y, z, M.mask);
-                    const int k0 = M.start[b], k1 = M.start[b + 1];
-                    if (k0 >= k1) continue;
-                    // the next record is in flight while this one is tested
-                    float4 nxt = M.spos[k0];
-                    for (int kk = k0; kk < k1; kk++) {
-                        const f3 pos = f3of(nxt);
-                        if (kk + 1 < k1) nxt = M.spos[kk + 1];
-                        int px, py, pz;
-                        photon_cell(pos, org, M.inv_cell, px, py, pz);
-                        if (px != x || py != y || pz != z) continue;
-                        float d2 = length_sq(pos - p);
-                        if (d2 > max_r2) continue;
-                        heap_insert<S>(h, count, kk, d2);
+                const int xa = face ? max(cx - ring, 0) : cx - ring, xb = min(cx + ring, tx);
+                for (int x0 = xa; x0 <= xb; x0 += 4 * xstep) {
+                    int c0[4], c1[4];
+                    float md[4];
+                    float4 first[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const int x = x0 + j * xstep;
+                        const float dx = axis_d(org.x + (float)x * M.cell, p.x);
+                        md[j] = (dx * dx + dy2) + dz2;
+                        c0[j] = c1[j] = 0;
+                        if (x >= 0 && x <= xb && !(md[j] > max_r2)) {
+                            const uint32_t b = photon_bucket(x, y, z, M.mask);
+                            c0[j] = M.start[b];
+                            c1[j] = M.start[b + 1];
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (c0[j] < c1[j]) first[j] = M.spos[c0[j]];
+                    for (int j = 0; j < 4; j++) {
+                        const int k0 = j == 0 ? c0[0] : j == 1 ? c0[1] : j == 2 ? c0[2] : c0[3];
+                        const int k1 = j == 0 ? c1[0] : j == 1 ? c1[1] : j == 2 ? c1[2] : c1[3];
+                        const float md2 = j == 0 ? md[0] : j == 1 ? md[1] : j == 2 ? md[2] : md[3];
+                        const int x = x0 + j * xstep;
+                        if (k0 >= k1) continue;
+                        if (count >= kGatherK && md2 >= h[0].x) continue;
+                        // the next record is in flight while this one is tested
+                        float4 nxt = j == 0 ? first[0] : j == 1 ? first[1] : j == 2 ? first[2] : first[3];
+                        for (int kk = k0; kk < k1; kk++) {
+                            const f3 pos = f3of(nxt);
+                            if (kk + 1 < k1) nxt = M.spos[kk + 1];
+                            int px, py, pz;
+                            photon_cell(pos, org, M.inv_cell, px, py, pz);
+                            if (px != x || py != y || pz != z) continue;
+                            float d2 = length_sq(pos - p);
+                            if (d2 > max_r2) continue;
+                            heap_insert<S>(h, count, kk, d2);
+                        }
                     }
                 }
             }
+        }
         float reach = (float)ring * M.cell;
         if (count >= kGatherK && h[0].x <= reach * reach) break;
         if (reach > M.max_r) break;

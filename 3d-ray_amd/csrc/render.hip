@@ -3258,7 +3258,7 @@ static int photon_pass(rt_ctx* ctx, const rt_scene* sc, const DevScene& S, int b
     size_t o_cnt = lay(4ull * nbmax), o_start = lay(4ull * (nbmax + 1));
     size_t o_hist = lay(4 * hist_n), o_hscan = lay(4 * hist_n);
     size_t o_bsum = lay(4ull * ((std::max(hist_n, (size_t)std::max(ntot, nbmax)) + kScanTile - 1) / kScanTile + 2));
-    size_t o_part = lay(16 * 256), o_org = lay(16), o_ovf = lay(16);
+    size_t o_part = lay(16 * 256), o_org = lay(32), o_ovf = lay(16);
     (void)tiles_max;
     if (need > ctx->ph_bytes) {
         if (ctx->ph_mem) hipFree(ctx->ph_mem);
@@ -3303,8 +3303,10 @@ static int photon_pass(rt_ctx* ctx, const rt_scene* sc, const DevScene& S, int b
     const float cell = std::max(cell_size, 1e-6f);
     GridParams G{cell, 1.0f / cell, (uint32_t)(nb - 1), n};
     int pb = std::min(256, (n + 255) / 256);
-    hipLaunchKernelGGL(k_min3, dim3(pb), dim3(256), 0, st, cp, n, part);
-    hipLaunchKernelGGL(k_min3, dim3(1), dim3(256), 0, st, part, pb, org);
+    hipLaunchKernelGGL(k_bound3<false>, dim3(pb), dim3(256), 0, st, cp, n, part);
+    hipLaunchKernelGGL(k_bound3<false>, dim3(1), dim3(256), 0, st, part, pb, org);
+    hipLaunchKernelGGL(k_bound3<true>, dim3(pb), dim3(256), 0, st, cp, n, part);
+    hipLaunchKernelGGL(k_bound3<true>, dim3(1), dim3(256), 0, st, part, pb, org + 1);
     HIP_TRY(hipMemsetAsync(cnt, 0, 4ull * nb, st));
     hipLaunchKernelGGL(k_photon_keys, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, cp, org, G, k0, v0, cnt);
     // stable LSD radix sort of (bucket, photon index)
@@ -3343,6 +3345,7 @@ static int photon_pass(rt_ctx* ctx, const rt_scene* sc, const DevScene& S, int b
     M.start = start;
     M.idx = vin;
     M.origin = org;
+    M.top = org + 1;
     M.cell = G.cell;
     M.inv_cell = G.inv_cell;
     M.mask = G.mask;
