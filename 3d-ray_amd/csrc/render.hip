@@ -1124,9 +1124,10 @@ __global__ void __launch_bounds__(kBlock) k_raygen(JOBS jobs, PathBufs P, int n,
 // scratch (PRIV); chosen per context.
 // Single flat scenes build for 8 waves/SIMD (64 VGPRs, 2 spilled; 2.6 %
 // faster than the 7-wave build), batches of flat scenes for 7; the
-// wrapper-entry traversal takes the registers it needs (3-4 waves).
+// wrapper-entry traversal for 5 (96 VGPRs; unbounded it takes 119, and the
+// 64-instance 960x540 frame 2.68 instead of 2.49 ms a launch).
 template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
-__global__ void __launch_bounds__(kWg, XF ? 1 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
+__global__ void __launch_bounds__(kWg, XF ? 5 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
     k_trace(JOBS jobs, PathBufs P) {
     __shared__ uint2 lds_stk[PRIV ? 1 : SD * kWg];
     __shared__ ChunkLds<kWaves, kChunkMax> lds;
@@ -2447,7 +2448,7 @@ __device__ __forceinline__ bool shadow_entry(const PathBufs& P, int maxs, int64_
 }
 
 template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
-__global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_shadow(JOBS jobs, PathBufs P, int maxs) {
+__global__ void __launch_bounds__(kBlock, XF ? 5 : 7) k_shadow(JOBS jobs, PathBufs P, int maxs) {
     __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
     uint2 priv_stk[PRIV ? SD : 1];
     uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
@@ -2660,10 +2661,13 @@ __global__ void k_resolve(RParams R, FilmBufs F, float exposure) {
 }
 
 // rt_trace_primary / rt_trace_rays
-template <int SD>
-__global__ void __launch_bounds__(kBlock) k_trace_primary(DevScene S, RParams R, int n, int32_t* prim, float* to,
+template <int SD, bool XF, bool PRIV>
+__global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_trace_primary(DevScene S, RParams R, int n, int32_t* prim, float* to,
                                                           float* uo, float* vo) {
-    __shared__ uint2 stk[SD * kBlock];
+    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
+    uint2 priv_stk[PRIV ? SD : 1];
+    uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
+    constexpr int STRIDE = PRIV ? 1 : kBlock;
     int p = xcd_block() * kBlock + threadIdx.x;
     if (p >= n) return;
     int i, j, s;
@@ -2674,23 +2678,23 @@ __global__ void __launch_bounds__(kBlock) k_trace_primary(DevScene S, RParams R,
     HitOut h;
     TravCount tc{0u, 0u, 0u};
     for (int skip = 0;;) {
-        if (S.xf)
-            h = trace_closest<SD, kBlock, false, false, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o,
-                                                              d, kEps, kInfinity, &stk[threadIdx.x],
+        if (XF)
+            h = trace_closest<SD, STRIDE, false, false, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o,
+                                                              d, kEps, kInfinity, stk,
                                                               (uint32_t*)(prim + n), tc, S.xf);
         else
-            h = trace_closest<SD, kBlock, false>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d, kEps,
-                                                 kInfinity, &stk[threadIdx.x], (uint32_t*)(prim + n), tc);
+            h = trace_closest<SD, STRIDE, false>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d, kEps,
+                                                 kInfinity, stk, (uint32_t*)(prim + n), tc);
         if (h.entry < 0) break;
         if (!hit_cam_invisible(S, h.entry, h.chain)) break;
-        if (S.xf) {
+        if (XF) {
             f3 lo, ld;
             o = offset_origin(make_surf_w(S, h.entry, h.chain, o, d, h.t, h.u, h.v, lo, ld).p, d);
         } else o = offset_origin(o + h.t * d, d);
         if (++skip >= 8) break;
     }
     float hu, hv;
-    if (S.xf && h.entry >= 0) chain_ray(S.entries, S.xf, h.chain, o, d);
+    if (XF && h.entry >= 0) chain_ray(S.entries, S.xf, h.chain, o, d);
     report_uv(S.entries, h, o, d, hu, hv);
     prim[p] = h.entry < 0 ? -1 : __float_as_int(S.entries[h.entry].b.w);
     to[p] = h.entry < 0 ? 0.0f : h.t;
@@ -2698,24 +2702,27 @@ __global__ void __launch_bounds__(kBlock) k_trace_primary(DevScene S, RParams R,
     vo[p] = h.entry < 0 ? 0.0f : hv;
 }
 
-template <int SD>
-__global__ void __launch_bounds__(kBlock) k_trace_rays(DevScene S, const float* __restrict__ rays, int n, int32_t* prim,
+template <int SD, bool XF, bool PRIV>
+__global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_trace_rays(DevScene S, const float* __restrict__ rays, int n, int32_t* prim,
                                                        float* to, float* uo, float* vo) {
-    __shared__ uint2 stk[SD * kBlock];
+    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
+    uint2 priv_stk[PRIV ? SD : 1];
+    uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
+    constexpr int STRIDE = PRIV ? 1 : kBlock;
     int p = xcd_block() * kBlock + threadIdx.x;
     if (p >= n) return;
     const float* r = rays + 6 * (int64_t)p;
     TravCount tc{0u, 0u, 0u};
     f3 o = mk(r[0], r[1], r[2]), d = mk(r[3], r[4], r[5]);
     HitOut h;
-    if (S.xf) {
-        h = trace_closest<SD, kBlock, false, false, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d,
-                                                          kEps, kInfinity, &stk[threadIdx.x], (uint32_t*)(prim + n), tc,
+    if (XF) {
+        h = trace_closest<SD, STRIDE, false, false, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d,
+                                                          kEps, kInfinity, stk, (uint32_t*)(prim + n), tc,
                                                           S.xf);
         if (h.entry >= 0) chain_ray(S.entries, S.xf, h.chain, o, d);
     } else
-        h = trace_closest<SD, kBlock, false>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d, kEps,
-                                             kInfinity, &stk[threadIdx.x], (uint32_t*)(prim + n), tc);
+        h = trace_closest<SD, STRIDE, false>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d, kEps,
+                                             kInfinity, stk, (uint32_t*)(prim + n), tc);
     float hu, hv;
     report_uv(S.entries, h, o, d, hu, hv);
     prim[p] = h.entry < 0 ? -1 : __float_as_int(S.entries[h.entry].b.w);
@@ -2726,27 +2733,30 @@ __global__ void __launch_bounds__(kBlock) k_trace_rays(DevScene S, const float* 
 
 // Occlusion queries (rt_occluded): the any-hit traversal the shadow kernel
 // runs for opaque scenes, on caller-given segments.
-template <int SD>
-__global__ void __launch_bounds__(kBlock) k_occluded(DevScene S, const float* __restrict__ rays, int n, int32_t* occ) {
-    __shared__ uint2 stk[SD * kBlock];
+template <int SD, bool XF, bool PRIV>
+__global__ void __launch_bounds__(kBlock, XF ? 4 : 7) k_occluded(DevScene S, const float* __restrict__ rays, int n, int32_t* occ) {
+    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kBlock];
+    uint2 priv_stk[PRIV ? SD : 1];
+    uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
+    constexpr int STRIDE = PRIV ? 1 : kBlock;
     int p = xcd_block() * kBlock + threadIdx.x;
     if (p >= n) return;
     const float* r = rays + 8 * (int64_t)p;
     f3 o = mk(r[0], r[1], r[2]), d = mk(r[3], r[4], r[5]);
     bool b;
-    if (S.nodes4) {
+    if (!XF && S.nodes4) {
         TravCount tc{0u, 0u, 0u};
-        b = trace_any4<SD, kBlock>(S.nodes4, S.entries, S.aux, S.top_start, S.top_count, o, d, r[6], r[7],
-                                   &stk[threadIdx.x], (uint32_t*)(occ + n), tc);
-    } else if (S.xf) {
+        b = trace_any4<SD, STRIDE>(S.nodes4, S.entries, S.aux, S.top_start, S.top_count, o, d, r[6], r[7],
+                                   stk, (uint32_t*)(occ + n), tc);
+    } else if (XF) {
         TravCount tc{0u, 0u, 0u};
-        b = trace_closest<SD, kBlock, false, true, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d,
-                                                         r[6], r[7], &stk[threadIdx.x], (uint32_t*)(occ + n), tc, S.xf)
+        b = trace_closest<SD, STRIDE, false, true, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d,
+                                                         r[6], r[7], stk, (uint32_t*)(occ + n), tc, S.xf)
                 .entry >= 0;
     } else {
         TravCount tc{0u, 0u, 0u};
-        b = trace_closest<SD, kBlock, false, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d, r[6], r[7],
-                                                   &stk[threadIdx.x], (uint32_t*)(occ + n), tc)
+        b = trace_closest<SD, STRIDE, false, true>(S.nodes, S.entries, S.aux, S.top_start, S.top_count, o, d, r[6], r[7],
+                                                   stk, (uint32_t*)(occ + n), tc)
                 .entry >= 0;
     }
     occ[p] = b ? 1 : 0;
@@ -2803,6 +2813,8 @@ struct rt_ctx {
     size_t io_bytes = 0;
     void* dn_mem = nullptr;                   // denoiser buffers (grow-only)
     size_t dn_bytes = 0;
+    void* qry_mem = nullptr;                  // rays and results of the ray queries (grow-only, at most kQueryKeep)
+    size_t qry_bytes = 0;
     char* scratch = nullptr;                  // this device's copy of rt::scratch (hipGetSymbolAddress)
 };
 
@@ -2865,6 +2877,25 @@ static int grow_buffer(rt_ctx* ctx, void** mem, size_t* have, size_t bytes, void
     return RT_OK;
 }
 int ctx_io_buffer(rt_ctx* ctx, size_t bytes, void** out) { return grow_buffer(ctx, &ctx->io_mem, &ctx->io_bytes, bytes, out); }
+// Device buffer of one ray query: the context's, or above kQueryKeep a one-off
+// allocation that query_release gives back.  A pair of 100 k-ray queries takes
+// 604 us, 730 with an allocation and a free in each.
+constexpr size_t kQueryKeep = (size_t)1 << 28;
+static int query_buffer(rt_ctx* ctx, size_t bytes, char** out) {
+    void* m = nullptr;
+    if (bytes <= kQueryKeep) {
+        const int rc = grow_buffer(ctx, &ctx->qry_mem, &ctx->qry_bytes, bytes, &m);
+        *out = (char*)m;
+        return rc;
+    }
+    const hipError_t e = hipMalloc(&m, bytes);
+    if (e != hipSuccess) return fail(ctx, RT_ERR_OUT_OF_MEMORY, hipGetErrorString(e));
+    *out = (char*)m;
+    return RT_OK;
+}
+static void query_release(rt_ctx* ctx, char* mem) {
+    if (mem != (char*)ctx->qry_mem) hipFree(mem);
+}
 int ctx_dn_buffer(rt_ctx* ctx, size_t bytes, void** out) { return grow_buffer(ctx, &ctx->dn_mem, &ctx->dn_bytes, bytes, out); }
 }  // namespace rt
 
@@ -2958,6 +2989,23 @@ static DevScene dev_view(const rt_scene* sc) {
         if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<J, 24, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__);      \
         else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<J, 32, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__); \
         else hipLaunchKernelGGL((KERNEL<J, 64, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__);                 \
+    } while (0)
+// Ray queries: kernels of their own for scenes with wrapper entries, and two
+// stack placements.  Up to kQueryLds rays every wave is resident with an LDS
+// stack too, and its pops answer sooner (100 k rays on 20 k triangles: 102
+// against 115 us); more rays take private stacks and twice the waves.
+constexpr int kQueryLds = 1 << 17;
+#define DISPATCH_SD_Q(sd, xf, n, KERNEL, grid, ...)                                                         \
+    do {                                                                                                    \
+        if (xf) DISPATCH_SD_QX(sd, true, true, KERNEL, grid, __VA_ARGS__);                                  \
+        else if ((n) > kQueryLds) DISPATCH_SD_QX(sd, false, true, KERNEL, grid, __VA_ARGS__);               \
+        else DISPATCH_SD_QX(sd, false, false, KERNEL, grid, __VA_ARGS__);                                   \
+    } while (0)
+#define DISPATCH_SD_QX(sd, X_, P_, KERNEL, grid, ...)                                                       \
+    do {                                                                                                    \
+        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<24, X_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);       \
+        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<32, X_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((KERNEL<64, X_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);                  \
     } while (0)
 #define DISPATCH_SD(sd, KERNEL, grid, ...)                                                       \
     do {                                                                                         \
@@ -3505,6 +3553,7 @@ void rt_destroy(rt_ctx* ctx) {
     if (ctx->adj_mem) hipFree(ctx->adj_mem);
     if (ctx->io_mem) hipFree(ctx->io_mem);
     if (ctx->dn_mem) hipFree(ctx->dn_mem);
+    if (ctx->qry_mem) hipFree(ctx->qry_mem);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -3650,14 +3699,14 @@ int rt_trace_primary(rt_ctx* ctx, const rt_scene* sc, const rt_settings* s, int3
     DevScene S = dev_view(sc);
     char* mem = nullptr;
     size_t bytes = (size_t)n * 16 + 64;
-    HIP_TRY(hipMalloc((void**)&mem, bytes));
+    if (int rc_ = query_buffer(ctx, bytes, &mem)) return rc_;
     int32_t* d_prim = (int32_t*)mem;
     float* d_t = (float*)(mem + 4 * (size_t)n + 16);
     float* d_u = d_t + n;
     float* d_v = d_u + n;
     hipMemsetAsync(mem, 0, bytes, ctx->stream);
     dim3 grid((unsigned)((n + kBlock - 1) / kBlock));
-    DISPATCH_SD(sc->stack_depth, k_trace_primary, grid, ctx->stream, S, R, (int)n, d_prim, d_t, d_u, d_v);
+    DISPATCH_SD_Q(sc->stack_depth, S.xf, n, k_trace_primary, grid, ctx->stream, S, R, (int)n, d_prim, d_t, d_u, d_v);
     hipError_t e = hipGetLastError();
     int32_t ovf = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&ovf, d_prim + n, 4, hipMemcpyDeviceToHost, ctx->stream);
@@ -3666,7 +3715,7 @@ int rt_trace_primary(rt_ctx* ctx, const rt_scene* sc, const rt_settings* s, int3
     if (e == hipSuccess && u) e = hipMemcpyAsync(u, d_u, 4 * n, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess && v) e = hipMemcpyAsync(v, d_v, 4 * n, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(mem);
+    query_release(ctx, mem);
     if (e != hipSuccess) return fail(ctx, RT_ERR_DEVICE, std::string("trace_primary: ") + hipGetErrorString(e));
     if (ovf) return fail(ctx, RT_ERR_INTERNAL, "traversal stack overflow");
     return RT_OK;
@@ -3680,21 +3729,21 @@ int rt_occluded(rt_ctx* ctx, const rt_scene* sc, const float* rays, int64_t num_
     int n = (int)num_rays;
     DevScene S = dev_view(sc);
     char* mem = nullptr;
-    HIP_TRY(hipMalloc((void**)&mem, (size_t)n * 32 + 4 * (size_t)(n + 4)));
+    if (int rc_ = query_buffer(ctx, (size_t)n * 32 + 4 * (size_t)(n + 4), &mem)) return rc_;
     float* d_rays = (float*)mem;
     int32_t* d_occ = (int32_t*)(mem + (size_t)n * 32);
     hipError_t e = hipMemcpyAsync(d_rays, rays, (size_t)n * 32, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(d_occ, 0, (size_t)(n + 4) * 4, ctx->stream);
     if (e == hipSuccess) {
         dim3 grid((unsigned)((n + kBlock - 1) / kBlock));
-        DISPATCH_SD(sc->stack_depth, k_occluded, grid, ctx->stream, S, d_rays, n, d_occ);
+        DISPATCH_SD_Q(sc->stack_depth, S.xf, n, k_occluded, grid, ctx->stream, S, d_rays, n, d_occ);
         e = hipGetLastError();
     }
     int32_t ovf = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&ovf, d_occ + n, 4, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(occluded, d_occ, 4 * (size_t)n, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(mem);
+    query_release(ctx, mem);
     if (e != hipSuccess) return fail(ctx, RT_ERR_DEVICE, std::string("occluded: ") + hipGetErrorString(e));
     if (ovf) return fail(ctx, RT_ERR_INTERNAL, "traversal stack overflow");
     return RT_OK;
@@ -3719,7 +3768,7 @@ int rt_occluded_noalloc(rt_ctx* ctx, const rt_scene* sc, const float* rays, int6
     if (e == hipSuccess) e = hipMemcpyAsync(d_rays, rays, (size_t)n * 32, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) {
         dim3 grid((unsigned)((n + kBlock - 1) / kBlock));
-        DISPATCH_SD(sc->stack_depth, k_occluded, grid, ctx->stream, S, d_rays, n, d_occ);
+        DISPATCH_SD_Q(sc->stack_depth, S.xf, n, k_occluded, grid, ctx->stream, S, d_rays, n, d_occ);
         e = hipGetLastError();
     }
     int32_t ovf = 0;
@@ -3741,7 +3790,7 @@ int rt_trace_rays(rt_ctx* ctx, const rt_scene* sc, const float* rays, int64_t nu
     DevScene S = dev_view(sc);
     char* mem = nullptr;
     size_t bytes = (size_t)n * (24 + 16) + 64;
-    HIP_TRY(hipMalloc((void**)&mem, bytes));
+    if (int rc_ = query_buffer(ctx, bytes, &mem)) return rc_;
     float* d_rays = (float*)mem;
     int32_t* d_prim = (int32_t*)(mem + (size_t)n * 24);
     float* d_t = (float*)(d_prim + n + 4);
@@ -3751,7 +3800,7 @@ int rt_trace_rays(rt_ctx* ctx, const rt_scene* sc, const float* rays, int64_t nu
     if (e == hipSuccess) e = hipMemsetAsync(d_prim, 0, (size_t)(n + 4) * 4, ctx->stream);
     if (e == hipSuccess) {
         dim3 grid((unsigned)((n + kBlock - 1) / kBlock));
-        DISPATCH_SD(sc->stack_depth, k_trace_rays, grid, ctx->stream, S, d_rays, n, d_prim, d_t, d_u, d_v);
+        DISPATCH_SD_Q(sc->stack_depth, S.xf, n, k_trace_rays, grid, ctx->stream, S, d_rays, n, d_prim, d_t, d_u, d_v);
         e = hipGetLastError();
     }
     int32_t ovf = 0;
@@ -3761,7 +3810,7 @@ int rt_trace_rays(rt_ctx* ctx, const rt_scene* sc, const float* rays, int64_t nu
     if (e == hipSuccess && u) e = hipMemcpyAsync(u, d_u, 4 * (size_t)n, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess && v) e = hipMemcpyAsync(v, d_v, 4 * (size_t)n, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(mem);
+    query_release(ctx, mem);
     if (e != hipSuccess) return fail(ctx, RT_ERR_DEVICE, std::string("trace_rays: ") + hipGetErrorString(e));
     if (ovf) return fail(ctx, RT_ERR_INTERNAL, "traversal stack overflow");
     return RT_OK;
