@@ -168,6 +168,8 @@ struct ManyJobs {
     int thin_film;              // some job's scene has a thin-film material (host-side launch choice)
     int hier;                   // some job's scene has an object hierarchy (host-side launch choice)
     int all_lights;             // every job samples all lights (host-side launch choice)
+    int any_hit;                // every job's scene is opaque to shadow rays and has the 4-wide BVH (likewise)
+    int max_depth;              // largest of the jobs' (host loop)
     __device__ __forceinline__ int job_of(const int32_t* job, int p) const { return job[p]; }
     __device__ __forceinline__ const DevScene& scene(int j) const { return J[j].S; }
     __device__ __forceinline__ const RParams& params(int j) const { return J[j].R; }
@@ -2419,32 +2421,121 @@ __device__ __forceinline__ void shadow_ray(const JOBS& jobs, const PathBufs& P, 
     });
 }
 
-// The thread's record of the shadow queue; false past its end.  Block b
-// works on the stripes that its XCD (b mod 8) filled, 64 entries of one
-// segment at a time.
+// A block's run of the shadow queue: entries [first, first + count) of
+// segment `seg` (count 0: none).  Block b works on the stripe that its XCD
+// (b mod 8) filled.  Runs are 64 entries, or where RUN asks for longer ones
+// (k_shadow_any) a 1024th of the stripe, at most kShadowRun, so that runs
+// are long where there is work for many rounds of waves and every CU has
+// some where there is not.
+constexpr int kShadowRun = 512;
+struct ShadowRun {
+    int64_t first;
+    int count, seg;
+};
+template <bool RUN>
 inline unsigned shadow_grid(const PathBufs& P, int maxs) {
     const int chunks = (P.n + P.chunk - 1) / P.chunk;
-    return (unsigned)(kStripes * ((int64_t)((chunks + kStripes - 1) / kStripes) * P.chunk / kBlock * maxs + maxs));
+    const int64_t cap = (int64_t)((chunks + kStripes - 1) / kStripes) * P.chunk * maxs;   // entries of a stripe
+    const int64_t runs = RUN ? std::min<int64_t>(cap / kBlock, std::max<int64_t>(4096, cap / kShadowRun)) : cap / kBlock;
+    return (unsigned)(kStripes * (runs + maxs + 1));
 }
-__device__ __forceinline__ bool shadow_entry(const PathBufs& P, int maxs, int64_t& sl) {
+template <bool RUN>
+__device__ __forceinline__ ShadowRun shadow_run(const PathBufs& P, int maxs) {
     const int lane = (int)threadIdx.x;
     const int stripes = shadow_stripes(maxs), nseg = (maxs <= kMaxSeg ? maxs : 1) * stripes;
-    // blocks of the lane's segment that are this block's stripe's (with fewer
-    // than 8 stripes the blocks of a stripe take turns)
     const int x = (int)(blockIdx.x % (unsigned)stripes), turn = (int)(blockIdx.x / (unsigned)stripes);
     const int count = lane < nseg && lane % stripes == x ? P.seg[lane * kSegStride] : 0;
-    int blocks = (count + kBlock - 1) / kBlock, incl = blocks;
+    int len = kBlock;
+    if (RUN) {
+        int t = count;
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        // with fewer than 8 stripes each is that much longer
+        len = min(kShadowRun, max(kBlock, t / (1024 * (kStripes / stripes)) / kBlock * kBlock));
+    }
+    const int runs = (count + len - 1) / len;
+    int incl = runs;
     for (int off = 1; off < 64; off <<= 1) {
         const int y = __shfl_up(incl, off, 64);
         if (lane >= off) incl += y;
     }
     const unsigned long long past = __ballot(incl > turn);
-    if (past == 0ull) return false;
-    const int s = __ffsll((long long)past) - 1;
-    const int i = (turn - (__shfl(incl, s, 64) - __shfl(blocks, s, 64))) * kBlock + lane;
-    if (i >= __shfl(count, s, 64)) return false;
-    sl = P.q_sh[(int64_t)P.q_seg * s + i];
+    if (past == 0ull) return ShadowRun{0, 0, 0};
+    const int s = __builtin_amdgcn_readfirstlane(__ffsll((long long)past) - 1);
+    const int at = (turn - (__shfl(incl, s, 64) - __shfl(runs, s, 64))) * len;
+    const int n = min(len, __shfl(count, s, 64) - at);
+    return ShadowRun{(int64_t)P.q_seg * s + __builtin_amdgcn_readfirstlane(at), __builtin_amdgcn_readfirstlane(n), s};
+}
+// The thread's record of the shadow queue; false past its end.
+__device__ __forceinline__ bool shadow_entry(const PathBufs& P, int maxs, int64_t& sl) {
+    const ShadowRun r = shadow_run<false>(P, maxs);
+    if ((int)threadIdx.x >= r.count) return false;
+    sl = P.q_sh[r.first + threadIdx.x];
     return true;
+}
+
+// Shadow rays of opaque scenes (every job's; any-hit on the 4-wide BVH): a
+// wave works through a run of the queue, a lane taking the next ray when its
+// own is answered.  Lanes are refilled once kRefill of them are idle, and a
+// wave tests nodes until fewer than kNodeLanes lanes have one, then the
+// leaves that have gathered.  Bound by each ray's chain of node and leaf
+// fetches; with a ray a lane a wave ran about four times its rays' mean.
+// 1080p x 64 frame of 1.31 M triangles, ms a frame: a ray a lane 93.5, here
+// 73.0 (refill at 8 / 16 / 24 idle 75.2 / 74.1 / 73.5; nodes down to 1 lane
+// 95.0, 16 75.5, 32 74.8, 40 76.6).  The closest-hit kernel keeps a ray a
+// lane: its camera rays are coherent as they are (54.6 ms, refilled 83.5).
+// It takes pools of kAnyRunPool slots: that frame with 33.5 / 16.8 / 8.4 / 4.2 /
+// 2.1 M slots spends 73 / 83 / 97 / 123 / 151 ms here against 94 / 98 / 104 / 110 /
+// 124 with a ray a lane, whose waves are more and shorter.
+constexpr int kRefill = 32, kNodeLanes = 24;
+constexpr int64_t kAnyRunPool = 1 << 23;
+template <class JOBS, int SD>
+__global__ void __launch_bounds__(kBlock, 8) k_shadow_any(JOBS jobs, PathBufs P, int maxs) {
+    uint32_t stk[SD];
+    const ShadowRun run = shadow_run<true>(P, maxs);
+    if (run.count == 0) return;
+    const int lane = (int)threadIdx.x;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    int next = 0;       // next entry of the run to start, wave-uniform
+    AnyRay r;
+    r.alive = false;
+    int32_t sl = 0, job = 0;
+    auto any4 = [&]() {
+        const DevScene& S = jobs.scene(job);
+        return Any4<SD>{S.nodes4, S.entries, S.aux, S.top_start, S.top_count, kEps, (uint32_t*)&P.counters[kCntOverflow]};
+    };
+    bool pend = false;  // the lane's ray has no result yet
+    for (;;) {
+        if (pend && !r.alive) {
+            const float4 c = r.blocked ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : P.sh_c[sl];
+            P.sh_r[sl] = make_float4(c.x, c.y, c.z, 0.0f);
+            pend = false;
+        }
+        const unsigned long long idle = __ballot(!r.alive);
+        const int free_lanes = __popcll(idle);
+        if (next < run.count) {
+            if (free_lanes >= kRefill) {
+                const int take = next + __popcll(idle & lt);
+                if (!r.alive && take < run.count) {
+                    sl = P.q_sh[run.first + take];
+                    if constexpr (!std::is_same<JOBS, OneJob>::value) job = jobs.job_of(P.job, (int)((int64_t)sl % P.n));
+                    const float4 o4 = P.sh_o[sl], d4 = P.sh_d[sl];
+                    any4().start(r, f3of(o4), f3of(d4), o4.w);
+                    pend = true;
+                }
+                next += free_lanes;
+            }
+        } else if (free_lanes == kBlock) {
+            break;
+        }
+        for (;;) {
+            const bool node = r.alive && !ref_is_leaf(r.cur);
+            const unsigned long long b = __ballot(node);
+            if (b == 0ull) break;
+            if (node) any4().node_step(r, stk);
+            if (__popcll(b) < kNodeLanes && __ballot(r.alive && ref_is_leaf(r.cur)) != 0ull) break;
+        }
+        if (r.alive && ref_is_leaf(r.cur)) any4().leaf_step(r, stk);
+    }
 }
 
 template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
@@ -3043,20 +3134,28 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                        int stack_depth, const DevScene* gather_scene, const DevPhotons* M, const WindowPlan& plan,
                        ACCUM accum, LoopTiming& tm) {
     const int64_t N = P.n;
-    bool thin_film, hier, rnd = false, all_lights;
+    bool thin_film, hier, rnd = false, all_lights, any_hit;
+    int max_depth;
     if constexpr (std::is_same<JOBS, OneJob>::value) {
         rnd = jobs.R.prng != 0;
+        max_depth = jobs.R.max_depth;
         all_lights = jobs.R.picked == 0;
         thin_film = jobs.S.thin_film != 0;
         hier = jobs.S.xf != nullptr;
+        any_hit = jobs.S.opaque_shadows && jobs.S.nodes4;
     } else {
+        max_depth = jobs.max_depth;
         thin_film = jobs.thin_film != 0;
         hier = jobs.hier != 0;
         all_lights = jobs.all_lights != 0;
+        any_hit = jobs.any_hit != 0;
     }
     const int pool_blocks = (int)((N + kBlock - 1) / kBlock);
     const int chunks = (int)((N + P.chunk - 1) / P.chunk);
-    const unsigned shadow_blocks = shadow_grid(P, maxs);
+    const unsigned shadow_blocks = shadow_grid<false>(P, maxs), any_blocks = shadow_grid<true>(P, maxs);
+    // runs with refilled lanes from kAnyRunPool slots; the instrumented and
+    // LDS-stack builds and smaller pools keep one ray a lane
+    any_hit = any_hit && !hier && !counting && ctx->priv_stack && N >= kAnyRunPool;
     size_t pbytes = sizeof(PartDev) * std::max<size_t>(plan.parts.size(), 1);
     if (pbytes > ctx->parts_bytes) {
         if (ctx->parts_mem) hipFree(ctx->parts_mem);
@@ -3141,7 +3240,14 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
             if (e) HIP_TRY(hipEventRecord(e[2], ctx->stream));
             if (gather_scene) hipLaunchKernelGGL(k_gather, dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, *gather_scene, Pw, *M);
             if (e) HIP_TRY(hipEventRecord(e[3], ctx->stream));
-            if (hier)
+            if (any_hit) {
+                if (stack_depth <= 24)
+                    hipLaunchKernelGGL((k_shadow_any<JOBS, 24>), dim3(any_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw, maxs);
+                else if (stack_depth <= 32)
+                    hipLaunchKernelGGL((k_shadow_any<JOBS, 32>), dim3(any_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw, maxs);
+                else
+                    hipLaunchKernelGGL((k_shadow_any<JOBS, 64>), dim3(any_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw, maxs);
+            } else if (hier)
                 DISPATCH_SD_X(JOBS, stack_depth, counting, k_shadow, dim3(shadow_blocks), kBlock, ctx->stream, jobs, Pw, maxs);
             else
                 DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_shadow, dim3(shadow_blocks), kBlock, ctx->stream,
@@ -3206,13 +3312,19 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
         // Once every sample of the window has been issued (known one batch
         // late), batches shrink to one iteration, so the window ends at most
         // one empty iteration after its last path instead of a whole batch.
+        // A window that fits the pool has started every sample, and each of
+        // its paths ends within max_depth iterations: the host enqueues that
+        // many and has no count to wait for (the 64 x 64 preview: 8 instead
+        // of 9 iterations and two waits).
+        int left = ws <= N ? std::max(max_depth, 1) : INT32_MAX;
         int nb[2] = {0, 0};   // iterations with timing events in each in-flight batch
         bool drain = false;
         for (int b = 0;; b++) {
             const int set = b & 1;
-            const int iters = drain ? 1 : kIterBatch;
+            const int iters = std::min(left, drain ? 1 : kIterBatch);
+            left -= iters;
             if (traced) tm.launches += iters;
-            if (gexec && !drain) {
+            if (gexec && iters == kIterBatch) {
                 HIP_TRY(hipGraphLaunch(gexec, ctx->stream));
                 nb[set] = 0;
             } else {
@@ -3225,8 +3337,16 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
             HIP_TRY(hipMemcpyAsync(&ctx->pinned[4 * set], &P.counters[kCntPend], 12, hipMemcpyDeviceToHost,
                                    ctx->stream));
             HIP_TRY(hipEventRecord(ctx->chk[set], ctx->stream));
-            if (b == 0) continue;
             const int prev = set ^ 1;
+            if (left == 0) {
+                HIP_TRY(hipEventSynchronize(ctx->chk[set]));
+                if (b > 0) collect(prev, nb[prev]);
+                collect(set, nb[set]);
+                if (ctx->pinned[4 * set + 1]) return fail(ctx, RT_ERR_INTERNAL, "traversal stack overflow");
+                if (ctx->pinned[4 * set] != 0) return fail(ctx, RT_ERR_INTERNAL, "paths left after max_depth iterations");
+                break;
+            }
+            if (b == 0) continue;
             HIP_TRY(hipEventSynchronize(ctx->chk[prev]));
             collect(prev, nb[prev]);
             if (ctx->pinned[4 * prev + 1]) return fail(ctx, RT_ERR_INTERNAL, "traversal stack overflow");
@@ -4510,11 +4630,13 @@ int rt_render_batch(rt_ctx* ctx, const rt_batch_job* jobs, int32_t n_jobs, int32
     hipEvent_t* ev = ctx->ev;
     HIP_TRY(hipEventRecord(ev[6], ctx->stream));
     LoopTiming tm;
-    ManyJobs many{(const JobDev*)ctx->jobs_mem, 0, 0, 1};
+    ManyJobs many{(const JobDev*)ctx->jobs_mem, 0, 0, 1, 1, 0};
     for (int j = 0; j < n_jobs; j++) {
         many.thin_film |= jd[j].S.thin_film;
         many.hier |= jd[j].S.xf != nullptr ? 1 : 0;
+        many.max_depth = std::max(many.max_depth, R[j].max_depth);
         if (R[j].picked) many.all_lights = 0;
+        if (!jd[j].S.opaque_shadows || !jd[j].S.nodes4) many.any_hit = 0;
     }
     auto accum = [&](const PartDev& pt) { launch_accum(ctx, R[pt.job], P, F[pt.job], pt); };
     for (const Segment& sg : segs) {

@@ -612,6 +612,141 @@ __device__ __forceinline__ bool trace_any4(const GNode4* __restrict__ nodes4, co
     return false;
 }
 
+// trace_any4 one step at a time, for waves that take a new ray into a lane as
+// soon as its ray is answered (the lanes of a wave need 11 node steps on
+// average and several times that at most, so a wave that waits for its
+// longest ray is three quarters idle).  Same tests, same order, same answer.
+struct AnyRay {
+    f3 o, d, inv;
+    float tmax;
+    uint32_t cur;       // node or leaf reference to visit
+    int sp;             // stack entries (references only)
+    uint32_t ti;        // next entry of the top-level list
+    bool alive, blocked;
+};
+
+template <int SD>
+struct Any4 {
+    const GNode4* __restrict__ nodes4;
+    const GEntry* __restrict__ entries;
+    const float4* __restrict__ aux;
+    uint32_t top_start, top_count;
+    float tmin;
+    uint32_t* overflow;
+
+    // The next nested BVH of the top-level list the ray enters; primitives on
+    // the way are tested.  Ends the ray when there is none.
+    __device__ __forceinline__ void next_top(AnyRay& r) const {
+        HitOut h;
+        TravCount tc{0u, 0u, 0u};
+        while (r.ti < top_count) {
+            const uint32_t e = top_start + r.ti++;
+            const float4 ea = entries[e].a, eb = entries[e].b, ec = entries[e].c;
+            const int32_t tag = tag_of(ea), kind = tag & 0xff, flags = tag >> 8;
+            float t = r.tmax, te;
+            if (kind != kBvh) {
+                if (!test_prim<false>(entries, ea, eb, ec, e, kind, flags, r.o, r.d, tmin, aux, t, h, tc)) continue;
+                r.blocked = true;
+                r.alive = false;
+                return;
+            }
+            if (!(flags & kEntryNoBox) && !slab(f3of(ea), f3of(eb), r.o, r.inv, tmin, r.tmax, te)) continue;
+            r.cur = (uint32_t)__float_as_int(ec.x);
+            return;
+        }
+        r.alive = false;
+    }
+    __device__ __forceinline__ void start(AnyRay& r, f3 o, f3 d, float tmax) const {
+        r.o = o;
+        r.d = d;
+        r.inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+        r.tmax = tmax;
+        r.sp = 0;
+        r.ti = 0u;
+        r.blocked = false;
+        r.alive = true;
+        next_top(r);
+    }
+    __device__ __forceinline__ void pop(AnyRay& r, const uint32_t* stk) const {
+        if (r.sp > 0) r.cur = stk[--r.sp];
+        else next_top(r);
+    }
+    // r.cur is an internal node
+    __device__ __forceinline__ void node_step(AnyRay& r, uint32_t* stk) const {
+        const GNode4 nd = nodes4[r.cur];
+        const float bx0[4] = {nd.mnx.x, nd.mnx.y, nd.mnx.z, nd.mnx.w}, bx1[4] = {nd.mxx.x, nd.mxx.y, nd.mxx.z, nd.mxx.w};
+        const float by0[4] = {nd.mny.x, nd.mny.y, nd.mny.z, nd.mny.w}, by1[4] = {nd.mxy.x, nd.mxy.y, nd.mxy.z, nd.mxy.w};
+        const float bz0[4] = {nd.mnz.x, nd.mnz.y, nd.mnz.z, nd.mnz.w}, bz1[4] = {nd.mxz.x, nd.mxz.y, nd.mxz.z, nd.mxz.w};
+        uint32_t ref[4] = {(uint32_t)nd.ch.x, (uint32_t)nd.ch.y, (uint32_t)nd.ch.z, (uint32_t)nd.ch.w};
+        float key[4];
+        int nh = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            float te;
+            const bool hk = slab(mk(bx0[k], by0[k], bz0[k]), mk(bx1[k], by1[k], bz1[k]), r.o, r.inv, tmin, r.tmax, te);
+            key[k] = hk ? te : __int_as_float(0x7f800000);
+            nh += hk ? 1 : 0;
+        }
+        auto cswap = [&](int a, int b) {
+            const bool sw = key[b] < key[a];
+            const float ka = key[a], kb = key[b];
+            const uint32_t ra = ref[a], rb = ref[b];
+            key[a] = sw ? kb : ka;
+            key[b] = sw ? ka : kb;
+            ref[a] = sw ? rb : ra;
+            ref[b] = sw ? ra : rb;
+        };
+        cswap(0, 1);
+        cswap(2, 3);
+        cswap(0, 2);
+        cswap(1, 3);
+        cswap(1, 2);
+        if (nh == 0) {
+            pop(r, stk);
+            return;
+        }
+        if (r.sp + nh - 1 > SD) {
+            *overflow = 1u;
+            r.alive = false;
+            return;
+        }
+        if (nh > 3) stk[r.sp++] = ref[3];
+        if (nh > 2) stk[r.sp++] = ref[2];
+        if (nh > 1) stk[r.sp++] = ref[1];
+        r.cur = ref[0];
+    }
+    // r.cur is a leaf
+    __device__ __forceinline__ void leaf_step(AnyRay& r, uint32_t* stk) const {
+        HitOut h;
+        TravCount tc{0u, 0u, 0u};
+        const uint32_t start = leaf_start(r.cur), cnt = leaf_count(r.cur);
+        for (uint32_t k = 0; k < cnt; k++) {
+            const uint32_t idx = start + k;
+            const float4 la = entries[idx].a, lb = entries[idx].b, lc = entries[idx].c;
+            const int32_t tag = tag_of(la), kind = tag & 0xff, flags = tag >> 8;
+            float t = r.tmax, te;
+            if (kind != kBvh) {
+                if (!test_prim<false>(entries, la, lb, lc, idx, kind, flags, r.o, r.d, tmin, aux, t, h, tc)) continue;
+                r.blocked = true;
+                r.alive = false;
+                return;
+            }
+            if (!(flags & kEntryNoBox) && !slab(f3of(la), f3of(lb), r.o, r.inv, tmin, r.tmax, te)) continue;
+            if (k + 1 < cnt) {
+                if (r.sp >= SD) {
+                    *overflow = 1u;
+                    r.alive = false;
+                    return;
+                }
+                stk[r.sp++] = leaf_ref(idx + 1, cnt - k - 1);
+            }
+            r.cur = (uint32_t)__float_as_int(lc.x);
+            return;
+        }
+        pop(r, stk);
+    }
+};
+
 // HitRecord.U/V of a reported hit: barycentrics for triangles, (alpha,
 // beta) for quads (both returned by the test), Sphere.GetSphereUV
 // (Sphere.cs:260-269) and InfinitePlane's tiled planar UV

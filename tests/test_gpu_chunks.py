@@ -86,3 +86,38 @@ def test_wide_nee_pool(gpu_ctx):
         sc.close()
     for k in ("beauty", "beauty_a", "beauty_b"):
         assert np.array_equal(getattr(a, k), getattr(b, k)), k
+
+
+@pytest.mark.parametrize("aovs", [False, True])
+def test_large_pool_shadow_runs(gpu_ctx, aovs):
+    # 8.9 M samples: the default pool's shadow waves work through runs of the
+    # queue and refill their lanes; a 1 M pool's keep a ray a lane
+    W, H = 1920, 929
+    desc = scenes.displaced_icosphere_scene(W, H, subdiv=4, sphere_lights=2)
+    sc = native.Scene(gpu_ctx, desc)
+    try:
+        a = _film(sc, W, H, 5, 0, aovs=aovs)
+        b = _film(sc, W, H, 5, 1 << 20, aovs=aovs)
+    finally:
+        sc.close()
+    assert a.beauty.mean() > 0
+    for k in ("beauty", "beauty_a", "beauty_b"):
+        assert np.array_equal(getattr(a, k), getattr(b, k)), k
+
+
+@pytest.mark.parametrize("name", ["cornell", "icosphere", "boxes"])
+def test_lds_stack_renders_the_same(gpu_ctx, name):
+    # the depth classes of the traversal stack (24, 32 and 64 entries)
+    desc = {"cornell": lambda: scenes.cornell(64, 48),
+            "icosphere": lambda: scenes.displaced_icosphere_scene(64, 48, subdiv=6),
+            "boxes": lambda: scenes.batch_scene(60000, 64, 48, 5, 2)}[name]()
+    sc = native.Scene(gpu_ctx, desc)
+    try:
+        a = _film(sc, 64, 48, 4, 0)
+        gpu_ctx.tune(traversal_stack=2)
+        b = _film(sc, 64, 48, 4, 0)
+    finally:
+        gpu_ctx.tune(traversal_stack=1)
+        sc.close()
+    for k in PLANES:
+        assert np.array_equal(getattr(a, k), getattr(b, k)), (name, k)
