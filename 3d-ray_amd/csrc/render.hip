@@ -3086,17 +3086,30 @@ static DevScene dev_view(const rt_scene* sc) {
 // stack too, and its pops answer sooner (100 k rays on 20 k triangles: 102
 // against 115 us); more rays take private stacks and twice the waves.
 constexpr int kQueryLds = 1 << 17;
-#define DISPATCH_SD_Q(sd, xf, n, KERNEL, grid, ...)                                                         \
-    do {                                                                                                    \
-        if (xf) DISPATCH_SD_QX(sd, true, true, KERNEL, grid, __VA_ARGS__);                                  \
-        else if ((n) > kQueryLds) DISPATCH_SD_QX(sd, false, true, KERNEL, grid, __VA_ARGS__);               \
-        else DISPATCH_SD_QX(sd, false, false, KERNEL, grid, __VA_ARGS__);                                   \
+#define DISPATCH_SD_Q(sd, xf, n, KERNEL, grid, ...)                                     \
+    do {                                                                                \
+        if (xf) DISPATCH_SD_QP(sd, true, KERNEL, grid, __VA_ARGS__);                    \
+        else if ((n) > kQueryLds) DISPATCH_SD_QP(sd, false, KERNEL, grid, __VA_ARGS__); \
+        else DISPATCH_SD_QL(sd, false, KERNEL, grid, __VA_ARGS__);                      \
     } while (0)
-#define DISPATCH_SD_QX(sd, X_, P_, KERNEL, grid, ...)                                                       \
-    do {                                                                                                    \
-        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<24, X_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);       \
-        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<32, X_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);  \
-        else hipLaunchKernelGGL((KERNEL<64, X_, P_>), grid, dim3(kBlock), 0, __VA_ARGS__);                  \
+// LDS stacks whatever the number of rays: these kernels need no scratch memory
+#define DISPATCH_SD_QL(sd, xf, KERNEL, grid, ...)                                       \
+    do {                                                                                \
+        if (xf) DISPATCH_SD_QLX(sd, true, KERNEL, grid, __VA_ARGS__);                   \
+        else DISPATCH_SD_QLX(sd, false, KERNEL, grid, __VA_ARGS__);                     \
+    } while (0)
+#define DISPATCH_SD_QLX(sd, X_, KERNEL, grid, ...)                                                             \
+    do {                                                                                                       \
+        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<24, X_, false>), grid, dim3(kBlock), 0, __VA_ARGS__);       \
+        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<32, X_, false>), grid, dim3(kBlock), 0, __VA_ARGS__);  \
+        else if ((sd) <= 48) hipLaunchKernelGGL((KERNEL<48, X_, false>), grid, dim3(kBlock), 0, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((KERNEL<64, X_, false>), grid, dim3(kBlock), 0, __VA_ARGS__);                  \
+    } while (0)
+#define DISPATCH_SD_QP(sd, X_, KERNEL, grid, ...)                                                              \
+    do {                                                                                                       \
+        if ((sd) <= 24) hipLaunchKernelGGL((KERNEL<24, X_, true>), grid, dim3(kBlock), 0, __VA_ARGS__);        \
+        else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<32, X_, true>), grid, dim3(kBlock), 0, __VA_ARGS__);   \
+        else hipLaunchKernelGGL((KERNEL<64, X_, true>), grid, dim3(kBlock), 0, __VA_ARGS__);                   \
     } while (0)
 #define DISPATCH_SD(sd, KERNEL, grid, ...)                                                       \
     do {                                                                                         \
@@ -3888,7 +3901,7 @@ int rt_occluded_noalloc(rt_ctx* ctx, const rt_scene* sc, const float* rays, int6
     if (e == hipSuccess) e = hipMemcpyAsync(d_rays, rays, (size_t)n * 32, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) {
         dim3 grid((unsigned)((n + kBlock - 1) / kBlock));
-        DISPATCH_SD_Q(sc->stack_depth, S.xf, n, k_occluded, grid, ctx->stream, S, d_rays, n, d_occ);
+        DISPATCH_SD_QL(sc->stack_depth, S.xf, k_occluded, grid, ctx->stream, S, d_rays, n, d_occ);
         e = hipGetLastError();
     }
     int32_t ovf = 0;

@@ -5,11 +5,15 @@ must equal rt_occluded's ray for ray, on two calls in a row (the second
 smaller, so stale contents of the first would show), and it refuses more
 segments than that array holds with a clear error."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 from helpers import random_triangles
+from hierarchy_cases import instanced_scene
 from raytracer import abi, scenes
 
 pytestmark = pytest.mark.gpu
@@ -71,3 +75,45 @@ def test_noalloc_refuses_more_than_its_staging(native):
     assert rc == abi.RT_OK
     sc.close()
     ctx.close()
+
+
+def _free_bytes(native):
+    """Free device memory, as the HIP runtime the library runs on counts it."""
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _grows(native, name):
+    """Device memory that the first large call takes in a fresh process,
+    where no kernel has made the runtime keep scratch memory yet."""
+    ctx = native.Context(0)
+    desc = {"mixed": lambda: random_triangles(4000, 23, planes=2), "instances": instanced_scene}[name]()
+    sc = native.Scene(ctx, desc)
+    rng = np.random.default_rng(3)
+    d = rng.normal(size=(300_000, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    segs = np.concatenate([rng.uniform(-3, 3, d.shape), d, np.tile([1e-4, 4.0], (len(d), 1))], 1).astype(np.float32)
+    if name == "mixed":
+        assert _noalloc(native, ctx, sc, segs[:64])[0] == abi.RT_OK   # code objects and staging are in place
+    before = _free_bytes(native)
+    rc, got = _noalloc(native, ctx, sc, segs)
+    assert rc == abi.RT_OK
+    grown = before - _free_bytes(native)
+    assert np.array_equal(got, sc.occluded(segs))
+    sc.close()
+    ctx.close()
+    return grown
+
+
+@pytest.mark.parametrize("name", ["mixed", "instances"])
+def test_noalloc_takes_no_device_memory(name):
+    # kernels with stacks in scratch would make the runtime allocate some at
+    # their first launch: above the ray queries' stack-placement line, and for
+    # scenes with wrapper entries
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.dirname(os.path.abspath(__file__))] + sys.path))
+    r = subprocess.run([sys.executable, "-c", "import sys, test_zz_no_alloc as t; from raytracer import native; "
+                        f"print('grown', t._grows(native, {name!r}))"], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert int(r.stdout.split()[-1]) <= 0, r.stdout
