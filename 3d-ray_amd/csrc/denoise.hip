@@ -35,6 +35,7 @@
 #include <cstring>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/rt3d.h"
@@ -166,12 +167,12 @@ __global__ void __launch_bounds__(kBlk) k_nlm_rows(const NlmJob* __restrict__ jo
 
 // Pass 2 of NlMeansCore.Filter for one chunk of offsets (NlMeansCore.cs:199-263),
 // per (job, pixel) in offset order; num/den carry over between chunks in
-// memory, the last chunk normalises (:268-281).  A thread takes kAccRows
-// pixels of a column: their 7-row patch sums share the plane's reads (10
-// instead of 28 for four), and the reads bound the kernel (1920x1080
-// prefilter: 10.5 ms with a pixel a thread, now 5.6).  A row outside the
-// plane adds 0, which leaves a sum that starts at +0 unchanged.
-constexpr int kAccRows = 4;
+// memory, the last chunk normalises (:268-281).  A thread takes ROWS pixels
+// of a column: their 7-row patch sums share the plane's reads (8 instead of
+// 14 for two), and the reads bound the kernel on a large film (1920x1080
+// prefilter: 10.5 ms with one row a thread, 4.8 with two; kAccWide).  A row
+// outside the plane adds 0, which leaves a sum that starts at +0 unchanged.
+template <int ROWS>
 __global__ void __launch_bounds__(kBlk) k_nlm_accum(const NlmJob* __restrict__ jobs, Geom G,
                                                     const float* __restrict__ dh, float invK2, int nf,
                                                     const float* __restrict__ feat, const float* __restrict__ fbw,
@@ -180,7 +181,7 @@ __global__ void __launch_bounds__(kBlk) k_nlm_accum(const NlmJob* __restrict__ j
     const NlmJob J = jobs[blockIdx.y];
     const int64_t n = (int64_t)G.w * G.h;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int x = (int)(i % G.w), yb = (int)(i / G.w) * kAccRows;
+    const int x = (int)(i % G.w), yb = (int)(i / G.w) * ROWS;
     if (yb >= G.h) return;
     const int64_t p0 = (int64_t)yb * G.w + x;
     const int tc = J.tc;
@@ -188,9 +189,9 @@ __global__ void __launch_bounds__(kBlk) k_nlm_accum(const NlmJob* __restrict__ j
     float* nm = num + (int64_t)blockIdx.y * 3 * n;
     float* dn = den + (int64_t)blockIdx.y * n;
     const float* dhj = dh + (int64_t)blockIdx.y * G.no * n;
-    float acc[kAccRows][3], dsum[kAccRows];
+    float acc[ROWS][3], dsum[ROWS];
 #pragma unroll
-    for (int r = 0; r < kAccRows; r++) {
+    for (int r = 0; r < ROWS; r++) {
         acc[r][0] = acc[r][1] = acc[r][2] = dsum[r] = 0.0f;
         if (!first && yb + r < G.h) {
             const int64_t p = p0 + (int64_t)r * G.w;
@@ -202,17 +203,17 @@ __global__ void __launch_bounds__(kBlk) k_nlm_accum(const NlmJob* __restrict__ j
     for (int ol = 0; ol < G.no; ol++) {
         int dx, dy, x0, x1, y0, y1;
         offset_region(G, G.o0 + ol, dx, dy, x0, x1, y0, y1);
-        if (x0 > x1 || y0 > y1 || x < x0 || x > x1 || yb > y1 || yb + kAccRows - 1 < y0) continue;
+        if (x0 > x1 || y0 > y1 || x < x0 || x > x1 || yb > y1 || yb + ROWS - 1 < y0) continue;
         const float* col = dhj + (int64_t)ol * n + x;
-        float v[kAccRows + 2 * P];
+        float v[ROWS + 2 * P];
 #pragma unroll
-        for (int k = 0; k < kAccRows + 2 * P; k++) {
+        for (int k = 0; k < ROWS + 2 * P; k++) {
             const int yy = yb - P + k;
             v[k] = yy >= y0 && yy <= y1 ? col[(int64_t)yy * G.w] : 0.0f;
         }
         const int nvec = ((x1 - x0 + 1) / kVecW) * kVecW;
 #pragma unroll
-        for (int r = 0; r < kAccRows; r++) {
+        for (int r = 0; r < ROWS; r++) {
             const int y = yb + r;
             if (y < y0 || y > y1) continue;
             const int cnt = min(y1, y + P) - max(y0, y - P) + 1;
@@ -234,7 +235,7 @@ __global__ void __launch_bounds__(kBlk) k_nlm_accum(const NlmJob* __restrict__ j
         }
     }
 #pragma unroll
-    for (int r = 0; r < kAccRows; r++) {
+    for (int r = 0; r < ROWS; r++) {
         if (yb + r >= G.h) break;
         const int64_t p = p0 + (int64_t)r * G.w;
         if (last) {
@@ -734,6 +735,12 @@ namespace {
         if (e_ != hipSuccess) return ctx_fail(ctx, RT_ERR_DEVICE, hipGetErrorString(e_)); \
     } while (0)
 
+// Pixels (times filterings of the batch) from which a k_nlm_accum thread takes
+// two rows; on smaller films a thread's serial chain over the offsets bounds
+// the kernel, and twice the threads with half the chain are faster.  Whole
+// NL-means calls, ms with 1 / 2 / 4 rows: 150x110 1.63 / 2.22 / 3.39, 480x360
+// 4.19 / 4.88 / 6.27, 640x480 7.45 / 7.12 / 9.61, 1280x720 21.7 / 20.3 / 24.0.
+constexpr int64_t kAccWide = 1 << 19;
 constexpr int kMaxPlanes = 768;   // dh planes per k_nlm_rows / k_nlm_accum pair (jobs x offsets)
 constexpr int kMaxJobs = 8;
 
@@ -802,10 +809,15 @@ int nlm(Pipe& Q, const std::vector<NlmJob>& jobs, int slot0, int R, float K, int
         Geom G{Q.w, Q.h, R, side, o0, std::min(chunk, offsets - o0)};
         const int64_t rows = (int64_t)Q.h * G.no;
         hipLaunchKernelGGL(k_nlm_rows, dim3(blocks(rows), nj), dim3(kBlk), 0, Q.st, dj, G, Q.dh);
-        const int64_t cols = (int64_t)Q.w * ((Q.h + kAccRows - 1) / kAccRows);
-        hipLaunchKernelGGL(k_nlm_accum, dim3(blocks(cols), nj), dim3(kBlk), 0, Q.st, dj, G,
-                           (const float*)Q.dh, invK2, nf, feat, (const float*)Q.bw, Q.num, Q.den, o0 == 0 ? 1 : 0,
-                           o0 + chunk >= offsets ? 1 : 0);
+        auto accum = [&](auto rows_a_thread) {
+            constexpr int kRows = decltype(rows_a_thread)::value;
+            const int64_t cols = (int64_t)Q.w * ((Q.h + kRows - 1) / kRows);
+            hipLaunchKernelGGL(k_nlm_accum<kRows>, dim3(blocks(cols), nj), dim3(kBlk), 0, Q.st, dj, G,
+                               (const float*)Q.dh, invK2, nf, feat, (const float*)Q.bw, Q.num, Q.den, o0 == 0 ? 1 : 0,
+                               o0 + chunk >= offsets ? 1 : 0);
+        };
+        if (Q.n * nj >= kAccWide) accum(std::integral_constant<int, 2>());
+        else accum(std::integral_constant<int, 1>());
     }
     return RT_OK;
 }

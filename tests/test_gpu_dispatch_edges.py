@@ -1,8 +1,8 @@
 """Sizes at which kernels change form: ray queries on both sides of the
 stack-placement threshold, gather points at the faces of the photons'
 bounding box (the k-nearest search visits only its cells), and films at the
-edges of the denoiser's tiles (4-row, 16- and 64-column runs, 16 x 16
-regression centres).  All bit-exact."""
+edges of the denoiser's tiles (16- and 64-column runs, 16 x 16 regression
+centres) and on both sides of its rows-a-thread line.  All bit-exact."""
 import numpy as np
 import pytest
 
@@ -63,3 +63,12 @@ def test_denoise_tile_edges(gpu_ctx, oracle, W, H, kind):
     buf = _film(gpu_ctx, scenes.cornell(W, H), W, H, 4)
     got = denoise.denoise(buf, denoise.DenoiserOptions(kind, "high"), gpu_ctx)
     _check(got, oracle.denoise(buf, kind, "high"), f"{kind} {W}x{H}")
+
+
+@pytest.mark.parametrize("W,H", [(297, 295), (513, 513)])
+def test_nlm_rows_a_thread(gpu_ctx, oracle, W, H):
+    # from 524,288 pixels times filterings (six in the prefilter, two in the
+    # main filter) a thread sums two rows: the prefilter only, then both
+    buf = _film(gpu_ctx, scenes.cornell(W, H), W, H, 2)
+    got = denoise.denoise(buf, denoise.DenoiserOptions("nlm", "fast"), gpu_ctx)
+    _check(got, oracle.denoise(buf, "nlm", "fast"), f"nlm {W}x{H}")
