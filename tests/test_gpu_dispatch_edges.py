@@ -72,3 +72,12 @@ def test_nlm_rows_a_thread(gpu_ctx, oracle, W, H):
     buf = _film(gpu_ctx, scenes.cornell(W, H), W, H, 2)
     got = denoise.denoise(buf, denoise.DenoiserOptions("nlm", "fast"), gpu_ctx)
     _check(got, oracle.denoise(buf, "nlm", "fast"), f"nlm {W}x{H}")
+
+
+@pytest.mark.parametrize("W,H", [(2, 9000), (2, 16420)])
+def test_nfor_offset_slices(gpu_ctx, oracle, W, H):
+    # 282 and 514 tiles of centres: the offsets in three slices, and in one
+    # (small films, as above, take up to 45)
+    buf = _film(gpu_ctx, scenes.cornell(W, H), W, H, 2)
+    got = denoise.denoise(buf, denoise.DenoiserOptions("nfor", "high"), gpu_ctx)
+    _check(got, oracle.denoise(buf, "nfor", "high"), f"nfor {W}x{H}")
