@@ -3250,9 +3250,13 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                     }
                 }
             }
+            // the shadow time starts at e[3], or at e[2] where no gather lies
+            // between: an event costs the stream 5 us
             if (e) HIP_TRY(hipEventRecord(e[2], ctx->stream));
-            if (gather_scene) hipLaunchKernelGGL(k_gather, dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, *gather_scene, Pw, *M);
-            if (e) HIP_TRY(hipEventRecord(e[3], ctx->stream));
+            if (gather_scene) {
+                hipLaunchKernelGGL(k_gather, dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, *gather_scene, Pw, *M);
+                if (e) HIP_TRY(hipEventRecord(e[3], ctx->stream));
+            }
             if (any_hit) {
                 if (stack_depth <= 24)
                     hipLaunchKernelGGL((k_shadow_any<JOBS, 24>), dim3(any_blocks), dim3(kBlock), 0, ctx->stream, jobs, Pw, maxs);
@@ -3287,7 +3291,7 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
             tm.trace += ms;
             hipEventElapsedTime(&ms, e[1], e[2]);
             tm.shade += ms;
-            hipEventElapsedTime(&ms, e[3], e[4]);
+            hipEventElapsedTime(&ms, gather_scene ? e[3] : e[2], e[4]);
             tm.shadow += ms;
         }
     };

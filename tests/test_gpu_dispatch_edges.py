@@ -81,3 +81,15 @@ def test_nfor_offset_slices(gpu_ctx, oracle, W, H):
     buf = _film(gpu_ctx, scenes.cornell(W, H), W, H, 2)
     got = denoise.denoise(buf, denoise.DenoiserOptions("nfor", "high"), gpu_ctx)
     _check(got, oracle.denoise(buf, "nfor", "high"), f"nfor {W}x{H}")
+
+
+@pytest.mark.parametrize("caustics", [False, True])
+def test_stage_times(gpu_ctx, caustics):
+    # the shadow stage's time starts behind the gather where there is one
+    sc = native.Scene(gpu_ctx, _small_caustics())
+    try:
+        st = native.Renderer(sc, 4, 8, enable_caustics=caustics, caustic_photons=20000 if caustics else 0).render(64, 48).stats
+    finally:
+        sc.close()
+    assert min(st.trace_ms, st.shade_ms, st.shadow_ms) > 0
+    assert st.trace_ms + st.shade_ms + st.shadow_ms < st.device_ms
