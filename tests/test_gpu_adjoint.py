@@ -225,3 +225,22 @@ def test_torch_autograd_wrapper(native, gpu_ctx):
         losses.append(float(l.detach()))
     print("losses", ["%.4f" % x for x in losses], flush=True)
     assert losses[-1] < 0.8 * losses[0]
+
+
+@pytest.mark.parametrize("size", [1, 3, 200])
+def test_texture_sizes_match_oracle_adjoint(native, oracle, gpu_ctx, size):
+    """Lanes of a wave with one footprint are summed before they reach the
+    texture: a texel for every lane, a few texels, and more footprints in a
+    wave than are gathered.  Bounds as above."""
+    W, H = 37, 29
+    rng = np.random.default_rng(size)
+    theta = rng.uniform(0.2, 0.8, (5, size, size)).astype(np.float32)
+    d = scenes.textured_icosphere_scene(W, H, subdiv=3, texture=theta)
+    r = _settings(native, native.Scene(gpu_ctx, d), 7, 3)
+    r.render(W, H)
+    db = rng.uniform(-1.0, 1.0, (3, H, W)).astype(np.float32)
+    g, _ = r.adjoint(W, H, db)
+    o = oracle.OracleScene(d).adjoint(r.settings, db)
+    err = np.linalg.norm(g - o) / np.linalg.norm(o)
+    print(f"{size}x{size} texture: relative L2 error {err:.3e}", flush=True)
+    assert err <= 1e-2
