@@ -339,7 +339,7 @@ __device__ __forceinline__ uint32_t xcd_block() { return xcd_remap(blockIdx.x, g
 // at a time: full waves whatever share of the slots is live, camera rays
 // beside camera rays, and no queue in memory.  k_trace runs four waves on up
 // to kChunkMax slots (a ray's cost varies: the waves take batches as they
-// get free); the bounce phase and k_retire run one wave on up to kChunkOne
+// get free; small pools: k_trace_one); the bounce phase and k_retire run one wave on up to kChunkOne
 // slots (their vertices cost about the same, and a lone wave waits for
 // nobody); the NEE phase runs four waves in pools of kNeeWide slots or more
 // (3.03 against 3.17 ms a launch at 33.5 M slots), one in smaller ones (40
@@ -1122,24 +1122,20 @@ __global__ void __launch_bounds__(kBlock) k_raygen(JOBS jobs, PathBufs P, int n,
     }
 }
 
-// Traversal stack placement: LDS (lane-interleaved) or the wave's private
-// scratch (PRIV); chosen per context.
-// Single flat scenes build for 8 waves/SIMD (64 VGPRs, 2 spilled; 2.6 %
-// faster than the 7-wave build), batches of flat scenes for 7; the
-// wrapper-entry traversal for 5 (96 VGPRs; unbounded it takes 119, and the
-// 64-instance 960x540 frame 2.68 instead of 2.49 ms a launch).
-template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
-__global__ void __launch_bounds__(kWg, XF ? 5 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
-    k_trace(JOBS jobs, PathBufs P) {
-    __shared__ uint2 lds_stk[PRIV ? 1 : SD * kWg];
-    __shared__ ChunkLds<kWaves, kChunkMax> lds;
+// Closest hits of a chunk's pending slots.  Traversal stack placement: LDS
+// (lane-interleaved) or the wave's private scratch (PRIV); chosen per context.
+template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF, int WAVES>
+__device__ __forceinline__ void trace_chunk(const JOBS& jobs, const PathBufs& P) {
+    __shared__ uint2 lds_stk[PRIV ? 1 : SD * WAVES * kBlock];
+    __shared__ ChunkLds<WAVES, WAVES == 1 ? kChunkOne : kChunkMax> lds;
     uint2 priv_stk[PRIV ? SD : 1];
     uint2* stk = PRIV ? priv_stk : &lds_stk[threadIdx.x];
-    constexpr int STRIDE = PRIV ? 1 : kWg;
+    constexpr int STRIDE = PRIV ? 1 : WAVES * kBlock;
     TravCount tc{0u, 0u, 0u};
-    const int base = chunk_base(P.wide);
+    const int chunk = WAVES == 1 ? P.chunk : P.wide;
+    const int base = chunk_base(chunk);
     // camera rays first, continuing paths after them
-    const ChunkList L = chunk_list(P.state, base, P.n, P.wide, lds, [](uint8_t st) {
+    const ChunkList L = chunk_list(P.state, base, P.n, chunk, lds, [](uint8_t st) {
         return st == kSlotFresh ? 0 : st == kSlotActive ? 1 : -1;
     });
     for (int t0 = L.take(); t0 < L.total(); t0 = L.take()) {
@@ -1178,6 +1174,29 @@ __global__ void __launch_bounds__(kWg, XF ? 5 : (std::is_same<JOBS, OneJob>::val
         });
     }
     if (COUNT) flush_counts(P.tcount, tc);
+}
+// Single flat scenes build for 8 waves/SIMD (64 VGPRs, 2 spilled; 2.6 %
+// faster than the 7-wave build), batches of flat scenes for 7; the
+// wrapper-entry traversal for 5 (96 VGPRs; unbounded it takes 119, and the
+// 64-instance 960x540 frame 2.68 instead of 2.49 ms a launch).
+template <class JOBS, int SD, bool COUNT, bool PRIV, bool XF = false>
+__global__ void __launch_bounds__(kWg, XF ? 5 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
+    k_trace(JOBS jobs, PathBufs P) {
+    trace_chunk<JOBS, SD, COUNT, PRIV, XF, kWaves>(jobs, P);
+}
+// Small pools: one wave a workgroup, on chunks of mostly 64 slots.  Four-wave
+// workgroups would leave CUs empty, and where every wave is resident a wave
+// of the live lanes of several rows takes longer than the rows side by side.
+// Above the line full waves are better.  Whole frames, ms with four waves and
+// with one, by pool slots.  64 to 146 instances: 12 k 4.14 / 3.69, 164 k 8.98 /
+// 8.38, 480 k 10.2 / 9.6, 1 M 12.8 / 19.3.  Icosphere of 82 k triangles: 21 k
+// 2.35 / 2.26, 240 k 3.26 / 3.22, 1 M 5.67 / 6.45; Cornell box: 128 k 1.27 /
+// 1.28, 480 k 2.43 / 2.47.
+constexpr int64_t kTraceWide = 1 << 18, kTraceWideXf = 1 << 19;
+template <class JOBS, int SD, bool XF>
+__global__ void __launch_bounds__(kBlock, XF ? 5 : (std::is_same<JOBS, OneJob>::value ? 8 : 7))
+    k_trace_one(JOBS jobs, PathBufs P) {
+    trace_chunk<JOBS, SD, false, true, XF, 1>(jobs, P);
 }
 
 // HitRecord.DpDu/DpDv an entry's hit writes (Triangle.cs:83-84, Quad.cs:79-80,
@@ -3081,6 +3100,13 @@ static DevScene dev_view(const rt_scene* sc) {
         else if ((sd) <= 32) hipLaunchKernelGGL((KERNEL<J, 32, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__); \
         else hipLaunchKernelGGL((KERNEL<J, 64, C_, true, true>), grid, dim3(bs), 0, __VA_ARGS__);                 \
     } while (0)
+// closest hits of small pools
+#define DISPATCH_SD_ONE(J, sd, X_, grid, ...)                                                             \
+    do {                                                                                                  \
+        if ((sd) <= 24) hipLaunchKernelGGL((k_trace_one<J, 24, X_>), grid, dim3(kBlock), 0, __VA_ARGS__);      \
+        else if ((sd) <= 32) hipLaunchKernelGGL((k_trace_one<J, 32, X_>), grid, dim3(kBlock), 0, __VA_ARGS__); \
+        else hipLaunchKernelGGL((k_trace_one<J, 64, X_>), grid, dim3(kBlock), 0, __VA_ARGS__);                 \
+    } while (0)
 // Ray queries: kernels of their own for scenes with wrapper entries, and two
 // stack placements.  Up to kQueryLds rays every wave is resident with an LDS
 // stack too, and its pops answer sooner (100 k rays on 20 k triangles: 102
@@ -3169,6 +3195,7 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
     // runs with refilled lanes from kAnyRunPool slots; the instrumented and
     // LDS-stack builds and smaller pools keep one ray a lane
     any_hit = any_hit && !hier && !counting && ctx->priv_stack && N >= kAnyRunPool;
+    const bool one_wave = N < (hier ? kTraceWideXf : kTraceWide) && !counting && ctx->priv_stack;   // closest hits
     size_t pbytes = sizeof(PartDev) * std::max<size_t>(plan.parts.size(), 1);
     if (pbytes > ctx->parts_bytes) {
         if (ctx->parts_mem) hipFree(ctx->parts_mem);
@@ -3182,10 +3209,16 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
     HIP_TRY(hipMemcpy(d_parts, plan.parts.data(), sizeof(PartDev) * plan.parts.size(), hipMemcpyHostToDevice));
     auto enqueue_iteration = [&](const PathBufs& Pw, hipEvent_t* e) -> int {
         if (traced) {
-            const dim3 grid(chunks);
+            const dim3 grid(chunks), wide_grid((unsigned)((N + P.wide - 1) / P.wide));
             if (e) HIP_TRY(hipEventRecord(e[0], ctx->stream));
-            if (hier) DISPATCH_SD_X(JOBS, stack_depth, counting, k_trace, dim3((unsigned)((N + P.wide - 1) / P.wide)), kWg, ctx->stream, jobs, Pw);
-            else DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_trace, dim3((unsigned)((N + P.wide - 1) / P.wide)), kWg, ctx->stream, jobs, Pw);
+            if (one_wave) {
+                if (hier) DISPATCH_SD_ONE(JOBS, stack_depth, true, grid, ctx->stream, jobs, Pw);
+                else DISPATCH_SD_ONE(JOBS, stack_depth, false, grid, ctx->stream, jobs, Pw);
+            } else if (hier) {
+                DISPATCH_SD_X(JOBS, stack_depth, counting, k_trace, wide_grid, kWg, ctx->stream, jobs, Pw);
+            } else {
+                DISPATCH_SD_C(JOBS, stack_depth, counting, ctx->priv_stack, k_trace, wide_grid, kWg, ctx->stream, jobs, Pw);
+            }
             if (e) HIP_TRY(hipEventRecord(e[1], ctx->stream));
             if (Pw.fp) DISPATCH_SD_C(JOBS, stack_depth, false, ctx->priv_stack, k_fp, dim3(pool_blocks), kBlock, ctx->stream, jobs, Pw);
             bool adj_replay = false;
@@ -3214,7 +3247,7 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
                     }
                 } else {
                     const bool wide = N >= kNeeWide;
-                    const dim3 ngrid(wide ? (unsigned)((N + P.wide - 1) / P.wide) : (unsigned)chunks);
+                    const dim3 ngrid = wide ? wide_grid : grid;
                     const dim3 nblk(wide ? kWg : kBlock);
 #define LAUNCH_NEE(W_, UL_)                                                                                          \
     do {                                                                                                             \

@@ -7,6 +7,7 @@ strips) follow the oracle."""
 import numpy as np
 import pytest
 
+from hierarchy_cases import instanced_scene
 from raytracer import abi, native, scenes
 
 pytestmark = pytest.mark.gpu
@@ -121,3 +122,23 @@ def test_lds_stack_renders_the_same(gpu_ctx, name):
         sc.close()
     for k in PLANES:
         assert np.array_equal(getattr(a, k), getattr(b, k)), (name, k)
+
+
+@pytest.mark.parametrize("kind", ["flat", "instances", "batch"])
+def test_closest_hits_of_small_and_large_pools(gpu_ctx, kind):
+    # 525,312 samples: closest hits by four-wave workgroups; the 64 k pool's
+    # by one-wave workgroups
+    W, H, spp = 1024, 513, 1
+    desc = instanced_scene(W, H) if kind == "instances" else _scene(W, H, 2)
+    sc = native.Scene(gpu_ctx, desc)
+    try:
+        if kind == "batch":
+            r = native.Renderer(sc, spp, 4)
+            a, b = (native.render_batch([(r, W, H), (r, W, H)], pool_paths=n)[0][1].buffers for n in (0, 1 << 16))
+        else:
+            a, b = (_film(sc, W, H, spp, n, aovs=False) for n in (0, 1 << 16))
+    finally:
+        sc.close()
+    assert a.beauty.mean() > 0
+    for k in ("beauty", "beauty_a", "beauty_b"):
+        assert np.array_equal(getattr(a, k), getattr(b, k)), k
