@@ -217,8 +217,10 @@ constexpr int kWcNext = 0, kWcRetire = 1, kWcRows = 2;
 // per light sample (ungrouped form: one) and per stripe of the workgroups
 // that fill it (at most 64 in all, a lane each), so the chunks' atomics
 // spread over that many lines; stripe x of segment j is size j * stripes + x.
-// The gather queue is the last.
-constexpr int kSegStride = 32, kSegGather = 64, kSegs = 65, kStripes = 8;
+// The gather queue has a stripe per XCD too, sizes kSegGather + x: with one
+// counter its atomics, one a chunk, took a NEE launch of 463 k slots from 45
+// to 83 us (400x300 x 4 caustics frame 4.79 against 4.48 ms).
+constexpr int kSegStride = 32, kSegGather = 64, kStripes = 8, kSegs = kSegGather + kStripes;
 RT_HD int shadow_stripes(int maxs) { return maxs <= 8 || maxs > kMaxSeg ? kStripes : maxs <= 16 ? 4 : 2; }
 constexpr int kIterBatch = 4;   // bounce iterations enqueued between host checks
 // Slot states.  Between iterations: idle, active (continues), fresh (a camera
@@ -252,7 +254,8 @@ struct PathBufs {
     int wide, chunk;            // slots per chunk of the four-wave and the one-wave kernels
     int32_t* q_sh;              // shadow queue: record indices, segment j stripe x from q_seg * (j * stripes + x)
     int q_seg;                  // entries a stripe of a segment can hold
-    int32_t* q_g;               // gather queue: slots with a request
+    int32_t* q_g;               // gather queue: slots with a request, stripe x from g_seg * x
+    int g_seg;                  // entries a stripe of it can hold
     int32_t* seg;               // queue sizes, size j at j * kSegStride
     int32_t* smask;             // per slot: light samples with a pending shadow ray (their number if maxs > kMaxSeg)
     int32_t* sid;               // sample of the window each path slot is tracing
@@ -2140,9 +2143,10 @@ __device__ __forceinline__ void queue_gathers(const PathBufs& P, int chunk, int 
         n += __popcll(b[k]);
     }
     if (n == 0) return;
+    const int x = (int)(blockIdx.x % (unsigned)kStripes);
     int at = 0;
-    if (lane == 0) at = atomicAdd(&P.seg[kSegGather * kSegStride], n);
-    at = __builtin_amdgcn_readfirstlane(at);
+    if (lane == 0) at = atomicAdd(&P.seg[(kSegGather + x) * kSegStride], n);
+    at = P.g_seg * x + __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
     for (int k = 0; k < kRows; k++) {
         if ((b[k] >> lane) & 1ull)
@@ -2301,7 +2305,7 @@ __global__ void __launch_bounds__(1024) k_scan(PathBufs P, int traced) {
     if (wid == 0) {
         long long t = P.seg[lane * kSegStride];
         P.seg[lane * kSegStride] = 0;
-        if (lane == 0) P.seg[kSegGather * kSegStride] = 0;
+        if (lane < kStripes) P.seg[(kSegGather + lane) * kSegStride] = 0;
         for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
         if (lane == 0 && t > 0) P.tcount[kTcShadowRays] += (unsigned long long)t;
     }
@@ -2359,11 +2363,10 @@ __device__ __forceinline__ void gather_slot(const DevScene& S, const PathBufs& P
 __global__ void __launch_bounds__(kBlock) k_gather(DevScene S, PathBufs P, DevPhotons M) {
     // the lane's heap of the k nearest photons, lane-interleaved
     __shared__ float2 lds_h[kGatherK * kBlock];
-    const int count = P.seg[kSegGather * kSegStride];
-    const uint32_t nb = (uint32_t)((count + kBlock - 1) / kBlock);
-    if (blockIdx.x >= nb) return;
-    const int i = (int)xcd_remap(blockIdx.x, nb, kXcdSlots / kBlock) * kBlock + (int)threadIdx.x;
-    if (i < count) gather_slot(S, P, M, P.q_g[i], &lds_h[threadIdx.x]);
+    // block b takes 64 entries of the stripe that its XCD (b mod 8) filled
+    const int x = (int)(blockIdx.x % (unsigned)kStripes);
+    const int i = (int)(blockIdx.x / (unsigned)kStripes) * kBlock + (int)threadIdx.x;
+    if (i < P.seg[(kSegGather + x) * kSegStride]) gather_slot(S, P, M, P.q_g[P.g_seg * x + i], &lds_h[threadIdx.x]);
 }
 
 // Transparent shadow walk (ShadowRay.Transmittance, ShadowRay.cs:59-158) of
@@ -3287,7 +3290,8 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
             // between: an event costs the stream 5 us
             if (e) HIP_TRY(hipEventRecord(e[2], ctx->stream));
             if (gather_scene) {
-                hipLaunchKernelGGL(k_gather, dim3(pool_blocks), dim3(kBlock), 0, ctx->stream, *gather_scene, Pw, *M);
+                hipLaunchKernelGGL(k_gather, dim3((unsigned)(kStripes * (Pw.g_seg / kBlock))), dim3(kBlock), 0,
+                                   ctx->stream, *gather_scene, Pw, *M);
                 if (e) HIP_TRY(hipEventRecord(e[3], ctx->stream));
             }
             if (any_hit) {
@@ -4093,16 +4097,21 @@ static int alloc_paths(rt_ctx* ctx, int64_t N, int64_t WS, int maxs, bool aovs, 
     const int chunk = chunk_one(N);
     const size_t nch = (size_t)(((N + chunk - 1) / chunk + 3) & ~(int64_t)3);   // row stride of the counts (int4 rows)
     size_t per_path = 8 * 16 + 8 * 4 + 4 + 16 + (aovs ? 5 * 16 : 0) + 4 * 16 * (size_t)maxs + 1 + 5 * 4 +
-                      (gather ? 69 : 0) + (fp ? 16 : 0) + (xf ? 16 : 0);
+                      (gather ? 65 : 0) + (fp ? 16 : 0) + (xf ? 16 : 0);
     // a stripe of a segment holds every chunk of its workgroups (times the
     // light samples in the ungrouped form)
     const int stripes = shadow_stripes(maxs);
     const int64_t stripe_slots = (((N + chunk - 1) / chunk + stripes - 1) / stripes) * chunk;
     const int64_t q_seg = stripe_slots * (maxs <= kMaxSeg ? 1 : maxs);
     const size_t q_all = (size_t)q_seg * stripes * (maxs <= kMaxSeg ? maxs : 1);
+    // a stripe of the gather queue holds every slot of its NEE workgroups
+    // (whole chunks, so a multiple of 64; four-wave chunks in wide pools)
+    auto stripe_of = [&](int64_t c) { return (((N + c - 1) / c + kStripes - 1) / kStripes) * c; };
+    const int64_t g_seg = std::max(stripe_of(chunk), N >= kNeeWide ? stripe_of(chunk_wide(N)) : 0);
     size_t per_sample = aovs ? 48 : 16;
     size_t need = (size_t)N * per_path + (size_t)WS * per_sample + 40 * 256 + 16384 +
-                  4 * kWcRows * nch + 4 * kSegStride * kSegs + 4 * q_all;
+                  4 * kWcRows * nch + 4 * kSegStride * kSegs + 4 * q_all +
+                  (gather ? 4 * (size_t)g_seg * kStripes : 0);
     if (need > ctx->path_bytes) {
         if (ctx->path_mem) hipFree(ctx->path_mem);
         ctx->path_mem = nullptr;
@@ -4159,7 +4168,8 @@ static int alloc_paths(rt_ctx* ctx, int64_t N, int64_t WS, int maxs, bool aovs, 
     P.res_l = (float4*)take(16 * WS);
     if (gather) {
         P.gflag = (uint8_t*)take(N);
-        P.q_g = (int32_t*)take(4 * N);
+        P.g_seg = (int)g_seg;
+        P.q_g = (int32_t*)take(4 * g_seg * kStripes);
         P.gq0 = (float4*)take(16 * N);
         P.gq1 = (float4*)take(16 * N);
         P.gq2 = (float4*)take(16 * N);

@@ -142,3 +142,19 @@ def test_closest_hits_of_small_and_large_pools(gpu_ctx, kind):
     assert a.beauty.mean() > 0
     for k in ("beauty", "beauty_a", "beauty_b"):
         assert np.array_equal(getattr(a, k), getattr(b, k)), k
+
+
+@pytest.mark.parametrize("sampler", ["sobol", "prng"])
+@pytest.mark.parametrize("W,H,spp,pools", [(65, 47, 5, (64, 1000, 0)), (1100, 1000, 4, (1 << 20, 0))])
+def test_caustic_films_of_any_pool(gpu_ctx, sampler, W, H, spp, pools):
+    # gather requests go through a queue with a stripe per XCD, filled by
+    # one-wave chunks and in pools of 4 M slots (Sobol) by four-wave ones
+    sc = native.Scene(gpu_ctx, scenes.caustics_scene(W, H, water_cells=20))
+    try:
+        films = [native.Renderer(sc, spp, 4, paths_in_flight=n, sampler=sampler, enable_caustics=True, caustic_photons=20000,
+                                 caustic_gather_radius=0.05).render(W, H).buffers for n in pools]
+    finally:
+        sc.close()
+    assert films[0].beauty.mean() > 0
+    for f in films[1:]:
+        assert np.array_equal(films[0].beauty, f.beauty)
