@@ -3111,15 +3111,23 @@ static DevScene dev_view(const rt_scene* sc) {
         else hipLaunchKernelGGL((k_trace_one<J, 64, X_>), grid, dim3(kBlock), 0, __VA_ARGS__);                 \
     } while (0)
 // Ray queries: kernels of their own for scenes with wrapper entries, and two
-// stack placements.  Up to kQueryLds rays every wave is resident with an LDS
-// stack too, and its pops answer sooner (100 k rays on 20 k triangles: 102
-// against 115 us); more rays take private stacks and twice the waves.
+// stack placements.  Pops of an LDS stack answer sooner, private stacks leave
+// room for more waves, and from about 130 k rays (a queue of 2048 waves) the
+// latter counts for more.  Whole calls, ms with LDS / private stacks:
+//                                  100 k          131 k          210 k
+//   closest hit, 20 k triangles    0.349 / 0.355  0.390 / 0.393  0.527 / 0.513
+//   closest hit, 328 k triangles   0.455 / 0.467  0.538 / 0.523  0.730 / 0.635
+//   occlusion, 328 k triangles     0.317 / 0.315  0.369 / 0.335  0.489 / 0.431
+//   closest hit, boxes (64-entry)  0.441 / 0.469  0.491 / 0.509  0.693 / 0.635
+//   closest hit, 64 instances      0.740 / 0.785  0.786 / 0.826  1.174 / 1.008
+// (the 64-entry LDS stacks leave 5 waves a CU, no more resident than 82 k
+// rays, and still win up to there.)
 constexpr int kQueryLds = 1 << 17;
 #define DISPATCH_SD_Q(sd, xf, n, KERNEL, grid, ...)                                     \
     do {                                                                                \
-        if (xf) DISPATCH_SD_QP(sd, true, KERNEL, grid, __VA_ARGS__);                    \
-        else if ((n) > kQueryLds) DISPATCH_SD_QP(sd, false, KERNEL, grid, __VA_ARGS__); \
-        else DISPATCH_SD_QL(sd, false, KERNEL, grid, __VA_ARGS__);                      \
+        if ((n) <= kQueryLds) DISPATCH_SD_QL(sd, xf, KERNEL, grid, __VA_ARGS__);        \
+        else if (xf) DISPATCH_SD_QP(sd, true, KERNEL, grid, __VA_ARGS__);               \
+        else DISPATCH_SD_QP(sd, false, KERNEL, grid, __VA_ARGS__);                      \
     } while (0)
 // LDS stacks whatever the number of rays: these kernels need no scratch memory
 #define DISPATCH_SD_QL(sd, xf, KERNEL, grid, ...)                                       \
