@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "rt_scene.h"
+#include "pixel_order.h"
 #include "shade.h"
 #include "adjoint.h"
 
@@ -109,17 +110,6 @@ struct RParams {
 struct PartDev {
     int job, pass0, off, npix, npass, width, pad[2];
 };
-
-// Pixel order of a window's samples: strips of 8 rows, column by column
-// inside a strip (64 consecutive pixels are an 8 x 8 tile); the last strip
-// takes the rows that are left.
-constexpr int kStripRows = 8;
-RT_HD int pixel_of_rank(int q, int W, int npix) {
-    const int strip = q / (kStripRows * W), y0 = strip * kStripRows;
-    const int r = q - y0 * W, left = npix / W - y0, h = left < kStripRows ? left : kStripRows;
-    const int x = r / h;
-    return (y0 + r - x * h) * W + x;
-}
 
 // Batch job on the device: its scene view and render parameters.
 struct JobDev {
