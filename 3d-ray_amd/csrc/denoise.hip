@@ -621,22 +621,23 @@ __global__ void __launch_bounds__(kBlk) k_scale(const float* src, int64_t n, con
 // rows and walks them kBoxCols columns at a time through LDS, whose loads and
 // stores are contiguous (1920 dependent strided loads a thread took 1.08 ms
 // for three 1920x1080 planes, now 0.36).
-constexpr int kBoxRows = 64, kBoxCols = 64, kBoxR = 4;   // kBoxR: largest radius
+constexpr int kBoxRows = 64, kBoxCols = 64;
 constexpr int kBoxWg = 512;   // eight waves move the tiles, the first sums
-__global__ void __launch_bounds__(kBoxWg) k_box_rows(const float* src, float* tmp, int w, int h, int r) {
-    constexpr int kIn = kBoxCols + 2 * kBoxR + 1;
+template <int r>
+__global__ void __launch_bounds__(kBoxWg) k_box_rows(const float* src, float* tmp, int w, int h) {
+    constexpr int kIn = kBoxCols + 2 * r + 1;
     __shared__ float in[kBoxRows][kIn], out[kBoxRows][kBoxCols + 1];
     const int yb = blockIdx.x * kBoxRows, y = yb + (int)threadIdx.x;
     const int64_t base = (int64_t)blockIdx.y * w * h;
     float run = 0.0f;
     for (int xb = 0; xb < w; xb += kBoxCols) {
         // columns [xb - r, xb + kBoxCols + r] of the wave's rows
-        const int c0 = xb - r, nc = kBoxCols + 2 * r + 1;
+        const int c0 = xb - r;
         __syncthreads();
 #pragma unroll 4
-        for (int i = threadIdx.x; i < kBoxRows * nc; i += kBoxWg) {
-            const int rr = i / nc, x = c0 + i % nc;
-            in[rr][i % nc] = yb + rr < h && x >= 0 && x < w ? src[base + (int64_t)(yb + rr) * w + x] : 0.0f;
+        for (int i = threadIdx.x; i < kBoxRows * kIn; i += kBoxWg) {
+            const int rr = i / kIn, x = c0 + i % kIn;
+            in[rr][i % kIn] = yb + rr < h && x >= 0 && x < w ? src[base + (int64_t)(yb + rr) * w + x] : 0.0f;
         }
         __syncthreads();
         if (threadIdx.x < kBoxRows && y < h) {
@@ -889,9 +890,10 @@ int percentile99(Pipe& Q, const float* x, float* result) {
 }
 
 // PlaneOps.BoxSmooth of `planes` consecutive planes (tmp: as many scratch planes)
-void box_smooth(Pipe& Q, const float* src, float* tmp, float* dst, int r, int planes) {
-    hipLaunchKernelGGL(k_box_rows, dim3((Q.h + kBoxRows - 1) / kBoxRows, planes), dim3(kBoxWg), 0, Q.st, src, tmp, Q.w,
-                       Q.h, r);   // r <= kBoxR
+template <int r>
+void box_smooth(Pipe& Q, const float* src, float* tmp, float* dst, int planes) {
+    hipLaunchKernelGGL(k_box_rows<r>, dim3((Q.h + kBoxRows - 1) / kBoxRows, planes), dim3(kBoxWg), 0, Q.st, src, tmp, Q.w,
+                       Q.h);
     hipLaunchKernelGGL(k_box_cols, dim3(blocks(Q.n), planes), dim3(kBlk), 0, Q.st, tmp, dst, Q.w, Q.h, r);
 }
 
@@ -978,9 +980,9 @@ int nfor(Pipe& Q, const NforBufs& B, const float* bA, const float* bB, const flo
         hipLaunchKernelGGL(k_mse_filtered, dim3(blocks(n)), dim3(kBlk), 0, Q.st,
                            (const float*)(B.reg + (int64_t)ki * 3 * n), (const float*)(B.reg + (int64_t)(nk + ki) * 3 * n),
                            bA, bB, bhv, n, margin, B.tmp + (int64_t)(ki + 1) * n);
-    box_smooth(Q, B.tmp, B.tmp2, B.mse, 4, ncand);
+    box_smooth<4>(Q, B.tmp, B.tmp2, B.mse, ncand);
     hipLaunchKernelGGL(k_indicator, dim3(blocks(n)), dim3(kBlk), 0, Q.st, (const float*)B.mse, ncand, n, B.tmp);
-    box_smooth(Q, B.tmp, B.tmp2, B.wts, 2, ncand);
+    box_smooth<2>(Q, B.tmp, B.tmp2, B.wts, ncand);
     hipLaunchKernelGGL(k_blend, dim3(blocks(n)), dim3(kBlk), 0, Q.st, (const float*)B.wts, (const float*)B.cand, ncand,
                        n, res);
     return RT_OK;
