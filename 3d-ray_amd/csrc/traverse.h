@@ -500,13 +500,46 @@ __device__ __forceinline__ bool slab_any(f3 mn_, f3 mx_, f3 o, f3 inv, float tmi
     return tx >= te;
 }
 
+// The children of a 4-wide node that the segment enters, nearest first (a
+// 5-exchange sorting network on their entry distances; misses sort last).
+__device__ __forceinline__ int hit_children4(const GNode4& nd, f3 o, f3 inv, float tmin, float tmax, uint32_t ref[4]) {
+    const float bx0[4] = {nd.mnx.x, nd.mnx.y, nd.mnx.z, nd.mnx.w}, bx1[4] = {nd.mxx.x, nd.mxx.y, nd.mxx.z, nd.mxx.w};
+    const float by0[4] = {nd.mny.x, nd.mny.y, nd.mny.z, nd.mny.w}, by1[4] = {nd.mxy.x, nd.mxy.y, nd.mxy.z, nd.mxy.w};
+    const float bz0[4] = {nd.mnz.x, nd.mnz.y, nd.mnz.z, nd.mnz.w}, bz1[4] = {nd.mxz.x, nd.mxz.y, nd.mxz.z, nd.mxz.w};
+    const uint32_t cref[4] = {(uint32_t)nd.ch.x, (uint32_t)nd.ch.y, (uint32_t)nd.ch.z, (uint32_t)nd.ch.w};
+    float key[4];
+    int nh = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        float te;
+        const bool hk = slab(mk(bx0[k], by0[k], bz0[k]), mk(bx1[k], by1[k], bz1[k]), o, inv, tmin, tmax, te);
+        key[k] = hk ? te : __int_as_float(0x7f800000);
+        ref[k] = cref[k];
+        nh += hk ? 1 : 0;
+    }
+    auto cswap = [&](int a, int b) {
+        const bool sw = key[b] < key[a];
+        const float ka = key[a], kb = key[b];
+        const uint32_t ra = ref[a], rb = ref[b];
+        key[a] = sw ? kb : ka;
+        key[b] = sw ? ka : kb;
+        ref[a] = sw ? rb : ra;
+        ref[b] = sw ? ra : rb;
+    };
+    cswap(0, 1);
+    cswap(2, 3);
+    cswap(0, 2);
+    cswap(1, 3);
+    cswap(1, 2);
+    return nh;
+}
+
 // Any-hit query on the 4-wide BVH (GNode4): is there a primitive hit with
 // t in [tmin, tmax]?  The answer equals the closest-hit traversal's
 // existence of a hit (every primitive whose boxes the segment enters is
 // tested; the visit order does not matter for a yes/no answer), with a
 // quarter of the dependent node fetches.  Hit children are visited nearest
-// first (a 5-exchange sorting network on their entry distances), which
-// finds occluders near the shading point sooner.
+// first, which finds occluders near the shading point sooner.
 template <int SD, int STRIDE, bool COUNT = false>
 __device__ __forceinline__ bool trace_any4(const GNode4* __restrict__ nodes4, const GEntry* __restrict__ entries,
                                            const float4* __restrict__ aux, uint32_t top_start, uint32_t top_count,
@@ -560,40 +593,8 @@ __device__ __forceinline__ bool trace_any4(const GNode4* __restrict__ nodes4, co
             } else {
                 const GNode4 nd = nodes4[cur];
                 if (COUNT) tc.node++;   // one 128-B node fetch
-                const float bx0[4] = {nd.mnx.x, nd.mnx.y, nd.mnx.z, nd.mnx.w};
-                const float by0[4] = {nd.mny.x, nd.mny.y, nd.mny.z, nd.mny.w};
-                const float bz0[4] = {nd.mnz.x, nd.mnz.y, nd.mnz.z, nd.mnz.w};
-                const float bx1[4] = {nd.mxx.x, nd.mxx.y, nd.mxx.z, nd.mxx.w};
-                const float by1[4] = {nd.mxy.x, nd.mxy.y, nd.mxy.z, nd.mxy.w};
-                const float bz1[4] = {nd.mxz.x, nd.mxz.y, nd.mxz.z, nd.mxz.w};
-                const uint32_t cref[4] = {(uint32_t)nd.ch.x, (uint32_t)nd.ch.y, (uint32_t)nd.ch.z, (uint32_t)nd.ch.w};
-                // hit children nearest first: entered in order of entry
-                // distance (a miss sorts last), the others pushed farthest first
-                float key[4];
                 uint32_t ref[4];
-                int nh = 0;
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    float te;
-                    const bool hk = slab(mk(bx0[k], by0[k], bz0[k]), mk(bx1[k], by1[k], bz1[k]), o, inv, tmin, closest, te);
-                    key[k] = hk ? te : __int_as_float(0x7f800000);
-                    ref[k] = cref[k];
-                    nh += hk ? 1 : 0;
-                }
-                auto cswap = [&](int a, int b) {
-                    const bool sw = key[b] < key[a];
-                    const float ka = key[a], kb = key[b];
-                    const uint32_t ra = ref[a], rb = ref[b];
-                    key[a] = sw ? kb : ka;
-                    key[b] = sw ? ka : kb;
-                    ref[a] = sw ? rb : ra;
-                    ref[b] = sw ? ra : rb;
-                };
-                cswap(0, 1);
-                cswap(2, 3);
-                cswap(0, 2);
-                cswap(1, 3);
-                cswap(1, 2);
+                const int nh = hit_children4(nd, o, inv, tmin, closest, ref);
                 if (nh > 0) {
                     // the pushes overflow exactly when the one-by-one pushes would
                     if (sp + nh - 1 > SD) { *overflow = 1u; return false; }
@@ -615,7 +616,8 @@ __device__ __forceinline__ bool trace_any4(const GNode4* __restrict__ nodes4, co
 // trace_any4 one step at a time, for waves that take a new ray into a lane as
 // soon as its ray is answered (the lanes of a wave need 11 node steps on
 // average and several times that at most, so a wave that waits for its
-// longest ray is three quarters idle).  Same tests, same order, same answer.
+// longest ray is three quarters idle).  Same tests, same order, same answer:
+// a change of the walk is made in both.
 struct AnyRay {
     f3 o, d, inv;
     float tmax;
@@ -674,33 +676,8 @@ struct Any4 {
     // r.cur is an internal node
     __device__ __forceinline__ void node_step(AnyRay& r, uint32_t* stk) const {
         const GNode4 nd = nodes4[r.cur];
-        const float bx0[4] = {nd.mnx.x, nd.mnx.y, nd.mnx.z, nd.mnx.w}, bx1[4] = {nd.mxx.x, nd.mxx.y, nd.mxx.z, nd.mxx.w};
-        const float by0[4] = {nd.mny.x, nd.mny.y, nd.mny.z, nd.mny.w}, by1[4] = {nd.mxy.x, nd.mxy.y, nd.mxy.z, nd.mxy.w};
-        const float bz0[4] = {nd.mnz.x, nd.mnz.y, nd.mnz.z, nd.mnz.w}, bz1[4] = {nd.mxz.x, nd.mxz.y, nd.mxz.z, nd.mxz.w};
-        uint32_t ref[4] = {(uint32_t)nd.ch.x, (uint32_t)nd.ch.y, (uint32_t)nd.ch.z, (uint32_t)nd.ch.w};
-        float key[4];
-        int nh = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            float te;
-            const bool hk = slab(mk(bx0[k], by0[k], bz0[k]), mk(bx1[k], by1[k], bz1[k]), r.o, r.inv, tmin, r.tmax, te);
-            key[k] = hk ? te : __int_as_float(0x7f800000);
-            nh += hk ? 1 : 0;
-        }
-        auto cswap = [&](int a, int b) {
-            const bool sw = key[b] < key[a];
-            const float ka = key[a], kb = key[b];
-            const uint32_t ra = ref[a], rb = ref[b];
-            key[a] = sw ? kb : ka;
-            key[b] = sw ? ka : kb;
-            ref[a] = sw ? rb : ra;
-            ref[b] = sw ? ra : rb;
-        };
-        cswap(0, 1);
-        cswap(2, 3);
-        cswap(0, 2);
-        cswap(1, 3);
-        cswap(1, 2);
+        uint32_t ref[4];
+        const int nh = hit_children4(nd, r.o, r.inv, tmin, r.tmax, ref);
         if (nh == 0) {
             pop(r, stk);
             return;
