@@ -1305,22 +1305,6 @@ __device__ __forceinline__ int32_t fold_shadows(const PathBufs& P, const RParams
     return flags & ~(0xff << kPfPendShift) & ~kPfPendInd;
 }
 
-// ADJ: the replay pass of the path-replay adjoint (rt_adjoint) — the same
-// shading plus, at textured Disney hits, the texture-gradient terms: NEE
-// records carry dBrdf/dp contracted with the pixel's adjoint weight (added by
-// k_adj_nee when the shadow ray is unoccluded), and a sampled bounce leaves
-// dF/dp / F (per channel) pending until the next shade, where the radiance
-// gathered after this vertex, D = (primal a0 + ai) - (a0 + ai so far), is
-// known (path replay backpropagation, Vicini, Speierer and Jakob 2021).
-//
-// PH = kPhNee leaves surface vertices of scattering materials in state
-// kSlotBounce with the vertex's throughput (medium weight applied), radiance
-// weight (segment weight applied), sampler dimension and pending-shadow
-// flags stored; PH = kPhBounce picks them up.  Sampler dimensions are drawn
-// in the same order either way.
-// RND: the PRNG sampler mode, fixed per kernel so the Sobol kernels carry no
-// code of the other mode.  UL: every job of the launch samples all lights
-// (no light pick), so the NEE light loop runs over a wave-uniform index.
 // The kernel's arguments as they lie in the argument segment.  Read through
 // a pointer the compiler cannot see through, so that a batch loads the fields
 // it uses with scalar loads where it uses them: hoisted out of the batch
@@ -1338,12 +1322,36 @@ __device__ __forceinline__ const ShadeArgs<JOBS>& shade_args() {
     asm volatile("" : "+s"(a));
     return *(const ShadeArgs<JOBS>*)a;
 }
+// A kernel of JOBS, PathBufs, int has its arguments at these offsets (each at
+// the next multiple of its alignment), as k_shade checks.
+template <class JOBS>
+constexpr bool shade_args_laid_out() {
+    constexpr size_t p = (sizeof(JOBS) + alignof(PathBufs) - 1) / alignof(PathBufs) * alignof(PathBufs);
+    constexpr size_t m = (p + sizeof(PathBufs) + alignof(int) - 1) / alignof(int) * alignof(int);
+    return offsetof(ShadeArgs<JOBS>, jobs) == 0 && offsetof(ShadeArgs<JOBS>, P) == p && offsetof(ShadeArgs<JOBS>, maxs) == m;
+}
 
 struct ShadeOut {
     int n_shadow;
     uint32_t smask;
     bool cont, bounce, disney_vtx, gather;
 };
+// ADJ: the replay pass of the path-replay adjoint (rt_adjoint) — the same
+// shading plus, at textured Disney hits, the texture-gradient terms: NEE
+// records carry dBrdf/dp contracted with the pixel's adjoint weight (added by
+// k_adj_nee when the shadow ray is unoccluded), and a sampled bounce leaves
+// dF/dp / F (per channel) pending until the next shade, where the radiance
+// gathered after this vertex, D = (primal a0 + ai) - (a0 + ai so far), is
+// known (path replay backpropagation, Vicini, Speierer and Jakob 2021).
+//
+// PH = kPhNee leaves surface vertices of scattering materials in state
+// kSlotBounceD or kSlotBounceO with the vertex's throughput (medium weight applied), radiance
+// weight (segment weight applied), sampler dimension and pending-shadow
+// flags stored; PH = kPhBounce picks them up.  Sampler dimensions are drawn
+// in the same order either way.
+// RND: the PRNG sampler mode, fixed per kernel so the Sobol kernels carry no
+// code of the other mode.  UL: every job of the launch samples all lights
+// (no light pick), so the NEE light loop runs over a wave-uniform index.
 template <class JOBS, bool ADJ, int PH, bool TF, bool RND, bool UL>
 __device__ __forceinline__ ShadeOut shade_slot(const JOBS& jobs, const PathBufs& P, int maxs, int p, bool active) {
     static_assert(!ADJ || PH == kPhAll, "the adjoint replay shades whole vertices");
@@ -2033,29 +2041,28 @@ __device__ __forceinline__ ShadeOut shade_slot(const JOBS& jobs, const PathBufs&
     return ShadeOut{n_shadow, smask, cont, bounce, disney_vtx, gather};
 }
 
-// Queues the chunk's shadow rays, all workgroup: the slots' masks (every
+// Queues the shadow rays of a one-wave chunk: the slots' masks (every
 // slot's: the NEE phase of a medium vertex may have left some) are read back,
 // counted per light sample and 64-slot row, one atomic per light sample takes
 // the chunk's range of its segment, and the records follow in slot order, so
 // a wave of k_shadow traces neighbouring paths' rays toward one light.  The
 // list memory is free by now.
-template <int WAVES, int MAX>
-__device__ __forceinline__ void queue_shadows(const PathBufs& P, int maxs, int base, ChunkLds<WAVES, MAX>& l) {
-    constexpr int kRows = MAX / (WAVES * kBlock);
-    const int lane = (int)__lane_id(), wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kBlock);
+template <int MAX>
+__device__ __forceinline__ void queue_shadows(const PathBufs& P, int maxs, int base, ChunkLds<1, MAX>& l) {
+    constexpr int kRows = MAX / kBlock;
+    const int lane = (int)threadIdx.x;
     const unsigned long long lt = (1ull << lane) - 1ull;
-    const int rows = P.chunk / (WAVES * kBlock), row0 = wid * rows;       // this wave's rows of the chunk
+    const int rows = P.chunk / kBlock;
     const bool grouped = maxs <= kMaxSeg;
     uint32_t m[kRows];
 #pragma unroll
     for (int k = 0; k < kRows; k++) {
-        const int p = base + (row0 + k) * kBlock + lane;
+        const int p = base + k * kBlock + lane;
         m[k] = k < rows && p < P.n ? (uint32_t)P.smask[p] : 0u;
     }
     uint32_t any = 0;
 #pragma unroll
     for (int k = 0; k < kRows; k++) any |= m[k];
-    static_assert(WAVES == 1, "one wave decides for the chunk");
     if (__ballot(any != 0u) == 0ull) return;
     const int stripes = shadow_stripes(maxs), x = (int)(blockIdx.x % (unsigned)stripes);
     if (grouped) {
@@ -2063,20 +2070,19 @@ __device__ __forceinline__ void queue_shadows(const PathBufs& P, int maxs, int b
         static_assert(MAX / kBlock * kMaxSeg <= MAX, "counts fit the list memory");
         uint16_t* cnt = l.q;
         int* start = l.start;
-        const int all = rows * WAVES;
         for (int j = 0; j < maxs; j++)
 #pragma unroll
             for (int k = 0; k < kRows; k++)
                 if (k < rows) {
                     const int c = __popcll(__ballot((m[k] >> j) & 1u));
-                    if (lane == 0) cnt[j * all + row0 + k] = (uint16_t)c;
+                    if (lane == 0) cnt[j * rows + k] = (uint16_t)c;
                 }
         __syncthreads();
         if ((int)threadIdx.x < maxs) {
             int t = 0;
-            for (int r = 0; r < all; r++) {
-                const int c = cnt[threadIdx.x * all + r];
-                cnt[threadIdx.x * all + r] = (uint16_t)t;
+            for (int r = 0; r < rows; r++) {
+                const int c = cnt[threadIdx.x * rows + r];
+                cnt[threadIdx.x * rows + r] = (uint16_t)t;
                 t += c;
             }
             start[threadIdx.x] = t > 0 ? atomicAdd(&P.seg[(threadIdx.x * stripes + x) * kSegStride], t) : 0;
@@ -2090,8 +2096,8 @@ __device__ __forceinline__ void queue_shadows(const PathBufs& P, int maxs, int b
                     const bool h = (m[k] >> j) & 1u;
                     const unsigned long long b = __ballot(h);
                     if (h)
-                        q[cnt[j * all + row0 + k] + __popcll(b & lt)] =
-                            (int32_t)((int64_t)j * P.n + base + (row0 + k) * kBlock + lane);
+                        q[cnt[j * rows + k] + __popcll(b & lt)] =
+                            (int32_t)((int64_t)j * P.n + base + k * kBlock + lane);
                 }
         }
     } else {
@@ -2114,7 +2120,7 @@ __device__ __forceinline__ void queue_shadows(const PathBufs& P, int maxs, int b
         for (int k = 0; k < kRows; k++)
             for (int i = 0; i < (int)m[k]; i++)
                 P.q_sh[(int64_t)P.q_seg * x + w0 + incl[k] - (int)m[k] + i] =
-                    (int32_t)((int64_t)i * P.n + base + (row0 + k) * kBlock + lane);
+                    (int32_t)((int64_t)i * P.n + base + k * kBlock + lane);
     }
 }
 
@@ -2148,6 +2154,9 @@ __device__ __forceinline__ void queue_gathers(const PathBufs& P, int chunk, int 
 template <class JOBS, int WPE, bool ADJ = false, int PH = kPhAll, bool TF = true, bool RND = false, bool UL = false,
           int WAVES = 1>
 __global__ void __launch_bounds__(WAVES * kBlock, WPE) k_shade(JOBS jobs, PathBufs P, int maxs) {
+    static_assert(std::is_same<decltype(&k_shade<JOBS, WPE, ADJ, PH, TF, RND, UL, WAVES>),
+                               void (*)(JOBS, PathBufs, int)>::value && shade_args_laid_out<JOBS>(),
+                  "shade_args reads the arguments as ShadeArgs");
     constexpr bool kFront = PH != kPhBounce, kBack = PH != kPhNee;
     static_assert(WAVES == 1 || PH == kPhNee, "chunk counts are one wave's");
     constexpr int kMax = WAVES == 1 ? kChunkOne : kChunkMax;
@@ -2433,8 +2442,8 @@ __device__ __forceinline__ void shadow_ray(const JOBS& jobs, const PathBufs& P, 
     });
 }
 
-// A block's run of the shadow queue: entries [first, first + count) of
-// segment `seg` (count 0: none).  Block b works on the stripe that its XCD
+// A block's run of the shadow queue: entries [first, first + count) of a
+// segment's stripe (count 0: none).  Block b works on the stripe that its XCD
 // (b mod 8) filled.  Runs are 64 entries, or where RUN asks for longer ones
 // (k_shadow_any) a 1024th of the stripe, at most kShadowRun, so that runs
 // are long where there is work for many rounds of waves and every CU has
@@ -2442,7 +2451,7 @@ __device__ __forceinline__ void shadow_ray(const JOBS& jobs, const PathBufs& P, 
 constexpr int kShadowRun = 512;
 struct ShadowRun {
     int64_t first;
-    int count, seg;
+    int count;
 };
 template <bool RUN>
 inline unsigned shadow_grid(const PathBufs& P, int maxs) {
@@ -2471,11 +2480,11 @@ __device__ __forceinline__ ShadowRun shadow_run(const PathBufs& P, int maxs) {
         if (lane >= off) incl += y;
     }
     const unsigned long long past = __ballot(incl > turn);
-    if (past == 0ull) return ShadowRun{0, 0, 0};
+    if (past == 0ull) return ShadowRun{0, 0};
     const int s = __builtin_amdgcn_readfirstlane(__ffsll((long long)past) - 1);
     const int at = (turn - (__shfl(incl, s, 64) - __shfl(runs, s, 64))) * len;
     const int n = min(len, __shfl(count, s, 64) - at);
-    return ShadowRun{(int64_t)P.q_seg * s + __builtin_amdgcn_readfirstlane(at), __builtin_amdgcn_readfirstlane(n), s};
+    return ShadowRun{(int64_t)P.q_seg * s + __builtin_amdgcn_readfirstlane(at), __builtin_amdgcn_readfirstlane(n)};
 }
 // The thread's record of the shadow queue; false past its end.
 __device__ __forceinline__ bool shadow_entry(const PathBufs& P, int maxs, int64_t& sl) {
@@ -3365,9 +3374,11 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
         // late), batches shrink to one iteration, so the window ends at most
         // one empty iteration after its last path instead of a whole batch.
         // A window that fits the pool has started every sample, and each of
-        // its paths ends within max_depth iterations: the host enqueues that
-        // many and has no count to wait for (the 64 x 64 preview: 8 instead
-        // of 9 iterations and two waits).
+        // its paths ends within max_depth iterations, so no more are enqueued.
+        // Up to two batches (max_depth 8) go out without a count to wait for
+        // (the 64 x 64 preview: 8 instead of 9 iterations and two waits);
+        // deeper windows go on one iteration at a time, which most leave
+        // before max_depth.
         int left = ws <= N ? std::max(max_depth, 1) : INT32_MAX;
         int nb[2] = {0, 0};   // iterations with timing events in each in-flight batch
         bool drain = false;
