@@ -2504,11 +2504,18 @@ __device__ __forceinline__ bool shadow_entry(const PathBufs& P, int maxs, int64_
 // 73.0 (refill at 8 / 16 / 24 idle 75.2 / 74.1 / 73.5; nodes down to 1 lane
 // 95.0, 16 75.5, 32 74.8, 40 76.6).  The closest-hit kernel keeps a ray a
 // lane: its camera rays are coherent as they are (54.6 ms, refilled 83.5).
-// It takes pools of kAnyRunPool slots: that frame with 33.5 / 16.8 / 8.4 / 4.2 /
-// 2.1 M slots spends 73 / 83 / 97 / 123 / 151 ms here against 94 / 98 / 104 / 110 /
-// 124 with a ray a lane, whose waves are more and shorter.
+// It takes pools of kAnyRunRays shadow records (slots x light samples a
+// vertex); with fewer a ray a lane is better, whose waves are more and shorter.
+// That frame with 33.5 / 16.8 / 8.4 / 4.2 / 2.1 M slots of 5 light samples spends 73
+// / 83 / 97 / 123 / 151 ms here against 94 / 98 / 104 / 110 / 124.  Whole 1500x940
+// frames of 1.3 k, 20 k and 328 k triangles, here / a ray a lane: 28 M slots x 5
+// 41.9 / 45.0, 49.1 / 52.3, 53.0 / 56.7 ms; 11 M x 5 24.2 / 24.2, 26.7 / 27.2, 29.3
+// / 29.5; 8.5 M x 5 20.8 / 20.4, 24.1 / 23.6, 25.3 / 24.9; 28 M x 1 (one light
+// picked) 38.8 / 38.6, 11 M x 1 22.9 / 22.4.  Batches: twelve scenes of 2 k triangles
+// 69.4 / 71.3, eight of 60 k 79.5 / 81.3 and 164 / 173 (16 and 32 M samples), eight of
+// 300 k 190 / 204.
 constexpr int kRefill = 32, kNodeLanes = 24;
-constexpr int64_t kAnyRunPool = 1 << 23;
+constexpr int64_t kAnyRunRays = 5ll << 23;
 template <class JOBS, int SD>
 __global__ void __launch_bounds__(kBlock, 8) k_shadow_any(JOBS jobs, PathBufs P, int maxs) {
     uint32_t stk[SD];
@@ -3202,9 +3209,9 @@ static int run_windows(rt_ctx* ctx, const JOBS& jobs, PathBufs P, int maxs, bool
     const int pool_blocks = (int)((N + kBlock - 1) / kBlock);
     const int chunks = (int)((N + P.chunk - 1) / P.chunk);
     const unsigned shadow_blocks = shadow_grid<false>(P, maxs), any_blocks = shadow_grid<true>(P, maxs);
-    // runs with refilled lanes from kAnyRunPool slots; the instrumented and
-    // LDS-stack builds and smaller pools keep one ray a lane
-    any_hit = any_hit && !hier && !counting && ctx->priv_stack && N >= kAnyRunPool;
+    // runs with refilled lanes from kAnyRunRays shadow records; the
+    // instrumented and LDS-stack builds and smaller pools keep a ray a lane
+    any_hit = any_hit && !hier && !counting && ctx->priv_stack && N * maxs >= kAnyRunRays;
     const bool one_wave = N < (hier ? kTraceWideXf : kTraceWide) && !counting && ctx->priv_stack;   // closest hits
     size_t pbytes = sizeof(PartDev) * std::max<size_t>(plan.parts.size(), 1);
     if (pbytes > ctx->parts_bytes) {
@@ -4279,15 +4286,16 @@ static int shadow_slots(const rt_settings* s, const HostScene& h) {
 // Renderer constructor arguments (Renderer.cs:300-378) as device parameters.
 // Default path pool: 32 M slots (~19 GB of path state with 5 shadow records
 // per path, 6.5 % of HBM).  Larger pools mean fewer bounce iterations per
-// frame (each with fixed scan/compaction/launch costs) and more rays per
-// launch over the same tree; the 1080p x 64 spp frame of the 1.31 M-triangle
-// scene renders at 397 / 397 / 412 / 381 / 388 Msamples/s with 16 / 28 / 32
-// / 36 / 40 M slots (the 32 M figure repeated on two boxes within 0.4 %).
+// frame and more rays per launch over the same tree: the 1080p x 64 spp frame
+// of the 1.31 M-triangle scene renders at 492 / 542 / 563 / 576 / 592 / 598 /
+// 612 Msamples/s with 8 / 16 / 24 / 32 / 40 / 48 / 64 M slots, but every other
+// render that fits keeps as much memory in its context.
 constexpr int64_t kDefaultPool = 1ll << 25;
 // rt_render_batch's default pool: 16 M slots.  Jobs of at least two pools of
-// samples run alone; with the 32 M pool more of a batch's jobs fall below
-// that and share windows, where their waves mix scenes (16-scene check:
-// batched/plain 0.978 at 16 M, 0.909 at 32 M).
+// samples run alone; the others share windows, where their waves mix scenes.
+// Plain over batched time of 16 scenes (10 k to 2 M triangles, up to 1080p x
+// 16): 0.922 / 0.917 / 0.926 / 0.935 / 0.902 with 8 / 16 / 24 / 32 / 48 M slots,
+// so within 2 % of each other, and 16 M takes half the memory of the default.
 constexpr int64_t kDefaultBatchPool = 1ll << 24;
 
 // Samples per window for a pool of `pool` slots.  A window's per-sample

@@ -158,3 +158,69 @@ def test_caustic_films_of_any_pool(gpu_ctx, sampler, W, H, spp, pools):
     assert films[0].beauty.mean() > 0
     for f in films[1:]:
         assert np.array_equal(films[0].beauty, f.beauty)
+
+
+def _mixed(W, H, samples):
+    """_scene's corner with nested meshes among the tree's leaves, and an
+    infinite plane at the top level beside the tree."""
+    b = scenes.SceneBuilder()
+    white = b.lambertian((0.7, 0.7, 0.7))
+    shiny = b.disney((0.6, 0.3, 0.2), roughness=0.3)
+    b.plane((0.0, 0.0, 0.0), (0.0, 1.0, 0.0), white)
+    b.quad((-3, 0, -3), (6, 0, 0), (0, 6, 0), white)
+    v, f = scenes.icosphere(3)
+    for k in range(5):
+        at = np.array([-1.6 + 0.8 * k, 0.45, 0.3 * (k % 2)])
+        if k % 2 == 0:
+            b.mesh(0.4 * v + at, f, shiny)
+        else:
+            b.sphere(at, 0.35, white)
+    for k in range(samples):
+        ang = 0.7 * k
+        b.area_light((2.0 * np.cos(ang), 3.0 + 0.1 * k, 2.0 * np.sin(ang)), (0.3, 0.0, 0.0), (0.0, 0.0, 0.3),
+                     intensity=12.0, shadow_samples=1)
+    return b.build(scenes.make_camera((0.0, 1.5, 5.0), (0.0, 0.7, 0.0), 45.0, W / H))
+
+
+@pytest.mark.parametrize("scene,samples", [("corner", 9), ("corner", 17), ("corner", 40), ("mixed", 5), ("mixed", 7)])
+def test_large_pool_shadow_runs_of_queue_forms(gpu_ctx, scene, samples):
+    # 8.4 M samples of at least 5 light samples: runs with refilled lanes, of 8,
+    # 4 and 2 stripes and of the ungrouped queue, and of rays that leave the
+    # tree for top-level entries and nested ones
+    W, H = 1024, 512
+    sc = native.Scene(gpu_ctx, (_scene if scene == "corner" else _mixed)(W, H, samples))
+    try:
+        a, b = (native.Renderer(sc, 16, 2, paths_in_flight=n).render(W, H).buffers for n in (0, 1 << 20))
+    finally:
+        sc.close()
+    assert a.beauty.mean() > 0
+    for k in ("beauty", "beauty_a", "beauty_b"):
+        assert np.array_equal(getattr(a, k), getattr(b, k)), k
+
+
+def test_wide_nee_pool_with_picked_lights(gpu_ctx):
+    W, H = 1024, 512
+    sc = native.Scene(gpu_ctx, _scene(W, H, 9))
+    try:
+        a, b = (native.Renderer(sc, 8, 4, light_sampling_strategy="power", paths_in_flight=n).render(W, H).buffers
+                for n in (0, 1 << 20))
+    finally:
+        sc.close()
+    assert a.beauty.mean() > 0
+    for k in ("beauty", "beauty_a", "beauty_b"):
+        assert np.array_equal(getattr(a, k), getattr(b, k)), k
+
+
+def test_large_batch_pool(gpu_ctx):
+    # 8.4 M samples of two scenes in one window: runs with refilled lanes
+    W, H = 1024, 512
+    scs = [native.Scene(gpu_ctx, _scene(W, H, 2)), native.Scene(gpu_ctx, _mixed(W, H, 6))]
+    try:
+        items = [(native.Renderer(sc, 8, 2), W, H) for sc in scs]
+        a, b = (native.render_batch(items, pool_paths=n)[0] for n in (0, 1 << 20))
+        for x, y in zip(a, b):
+            assert x.buffers.beauty.mean() > 0
+            assert np.array_equal(x.buffers.beauty, y.buffers.beauty)
+    finally:
+        for sc in scs:
+            sc.close()
