@@ -524,7 +524,11 @@ int rt_trace_primary(rt_ctx* ctx, const rt_scene* scene, const rt_settings* sett
  * collapsed from the binary one); the answer equals the existence of a
  * closest hit on [tmin, tmax].
  * Replaces: ShadowRay.Transmittance's occlusion test for opaque materials
- * (src/RayTracer/Rendering/ShadowRay.cs:59-158, BvhNode.Hit with the segment). */
+ * (src/RayTracer/Rendering/ShadowRay.cs:59-158, BvhNode.Hit with the segment).
+ * rt_trace_primary, rt_trace_rays and rt_occluded stage their rays and results
+ * in one device buffer of the context, which grows to the largest query so far
+ * (at most 256 MiB) and is held until rt_destroy; a query that needs more
+ * allocates its own and frees it before it returns. */
 int rt_occluded(rt_ctx* ctx, const rt_scene* scene, const float* rays, int64_t num_rays, int32_t* occluded);
 
 /* rt_occluded without device allocation.  No counterpart in the reference:
