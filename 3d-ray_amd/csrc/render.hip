@@ -311,19 +311,6 @@ constexpr int kBlock = 64;
 __device__ __forceinline__ int pf_cat(int32_t f) { return (f >> kPfCatShift) & 3; }
 __device__ __forceinline__ int pf_pend(int32_t f) { return (f >> kPfPendShift) & 0xff; }
 
-// XCD-aware block order: gfx950 dispatches consecutive workgroups round-robin
-// over its 8 XCDs; renumber so each XCD walks runs of `run` consecutive
-// blocks (neighbouring rays share BVH nodes in that XCD's L2) while the eight
-// stay side by side in the pool, so sky and object parts of the image load
-// them evenly (one eighth of the pool per XCD ran the 1080p frame in 349
-// instead of 298 ms).  Runs of 2048 slots.
-constexpr uint32_t kXcdSlots = 2048;
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb, uint32_t run) {
-    const uint32_t whole = nb / (8u * run) * (8u * run);
-    if (b >= whole) return b;   // the last, partial round keeps its order
-    const uint32_t x = b % 8u, i = b / 8u;
-    return (i / run * 8u + x) * run + i % run;
-}
 __device__ __forceinline__ uint32_t xcd_block() { return xcd_remap(blockIdx.x, gridDim.x, kXcdSlots / kBlock); }
 
 // ── chunks: the pool kernels' unit of work ───────────────────────────────
