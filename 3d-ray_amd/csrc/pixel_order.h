@@ -24,10 +24,11 @@ RT_HD int pixel_of_rank(int q, int W, int npix) {
 // side by side in the pool, so sky and object parts of the image load them
 // evenly (one eighth of the pool per XCD ran the 1080p frame in 349 instead of
 // 298 ms).  Runs of `longest` blocks (2048 slots), in small pools of a 64th of
-// an XCD's share, but a quarter of `longest` at least, and the XCDs change places from one eight of runs to the
-// next: in a fixed order an image whose strips are 4 or 8 runs long gives an
-// XCD the same columns of every strip (341x206 x 3 Cornell box, sky on both
-// sides: 1.77 ms, 1.53 with an eighth of the pool each, 1.54 here).
+// an XCD's share, but a quarter of `longest` at least, and the XCDs change
+// places from one eight of runs to the next: in a fixed order an image whose
+// strips are 4 or 8 runs long gives an XCD the same columns of every strip
+// (341x206 x 3 Cornell box, sky on both sides: 1.77 ms, 1.53 with an eighth of
+// the pool each, 1.54 here).
 constexpr uint32_t kXcdSlots = 2048;
 RT_HD uint32_t xcd_remap(uint32_t b, uint32_t nb, uint32_t longest) {
     const uint32_t share = nb / 512u, least = (longest + 3u) / 4u;

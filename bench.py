@@ -599,7 +599,8 @@ def main():
              "bytes_per_launch": round(bytes_per_launch), "avg_launch_ms": round(t_avg_s * 1000.0, 4),
              "launches_per_step": launches}
         if k == "shade":
-            r["note"] = "issue-bound (VALU, IEEE divisions): its HBM roofline is not its limit"
+            r["note"] = ("two kernels: the bounce phase is issue-bound (VALU, IEEE divisions), the NEE phase moves its light "
+                         "records at two thirds of the copy rate; the 352 B per event count neither's records")
         if ref_b is not None:
             r["reference_traversal"] = {
                 "bytes_per_launch": round(ref_b / max(launches, 1)),
