@@ -91,10 +91,11 @@ def test_wide_nee_pool(gpu_ctx):
 
 @pytest.mark.parametrize("aovs", [False, True])
 def test_large_pool_shadow_runs(gpu_ctx, aovs):
-    # 8.9 M samples: the default pool's shadow waves work through runs of the
-    # queue and refill their lanes; a 1 M pool's keep a ray a lane
+    # 8.9 M samples of five light samples: the default pool's shadow waves work
+    # through runs of the queue and refill their lanes; a 1 M pool's keep a ray
+    # a lane
     W, H = 1920, 929
-    desc = scenes.displaced_icosphere_scene(W, H, subdiv=4, sphere_lights=2)
+    desc = scenes.displaced_icosphere_scene(W, H, subdiv=4, sphere_lights=4)
     sc = native.Scene(gpu_ctx, desc)
     try:
         a = _film(sc, W, H, 5, 0, aovs=aovs)
